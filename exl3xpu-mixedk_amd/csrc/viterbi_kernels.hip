@@ -212,11 +212,12 @@ __device__ __forceinline__ int bp_lookup(const uint8_t* row, int j) {
 
 // --------------------------------------------------------------- forward DP
 // Whether the candidate arithmetic is issued grouped by opcode (see fwd_run):
-// measured faster for K >= 6, and for K = 4, 5 with T >= 2 sequences per
-// workgroup (K=4 +1.6 % with the wave priorities below); at T = 1 (the
-// column chain) K = 4 and 5 are 1-3 % faster ungrouped.
+// measured faster for K >= 4 (K=4 at T = 4 +1.6 %; at T = 1, with the units
+// of kPreUnits, the column chain K=4/5 402k/391k -> 406k/396k tiles/s) and for
+// K = 3 at T = 1 (372k -> 380k); K = 3 at T = 2 and K = 2 are 1-2 % faster in
+// the compiler's own order.
 template <int K, int T>
-constexpr bool kGroupOps = (K >= 6) || ((K == 4 || K == 5) && T >= 2);
+constexpr bool kGroupOps = (K >= 4) || (K == 3 && T == 1);
 
 // The same choice for the min-only steps.
 template <int K, int T>
@@ -291,6 +292,23 @@ constexpr bool kEarlyPair = (K == 4 && T >= 2);
 // chain at K=4 +1.5 %).
 template <int K, int T>
 constexpr bool kRematLane = (T == 1 && K <= 3);
+
+// Units (chunks of one group's candidates) whose squares fl(fl(f - x)^2) of
+// step i+1 a wave of a one-sequence workgroup computes at the end of step i,
+// before the barrier: they need the next target but no b, so waves that are
+// done early fill the issue slots that the step's last waves leave idle, and
+// after the barrier only the adds wait for the LDS round trip.  They run at
+// priority 0, one level below everything else of the step (kPrioBase).  The
+// 2560x4096 column chain at K = 3/4/5: 369k/395k/388k -> 380k/406k/396k
+// tiles/s with two units (one: 372k/400k/392k; three spill at K = 4, 5;
+// computed after the barrier instead: 371k/395k/394k).  K = 2 gains nothing
+// and K = 6, 7, whose units belong to one group, lose 2-3 % (382k -> 371k,
+// 368k -> 363k).  With more sequences per workgroup the other sequences'
+// work already fills those slots.
+template <int K, int T>
+constexpr int kPreUnits = (T == 1 && K >= 3 && K <= 5) ? 2 : 0;
+template <int K, int T>
+constexpr int kPrioBase = kPreUnits<K, T> > 0 ? 1 : 0;
 
 // Shared memory of one forward run over T sequences.
 template <int K, int T>
@@ -379,13 +397,35 @@ __device__ __forceinline__ void fwd_run(
     // whatever the order), half an instruction per candidate against the
     // key path's one v_min_f64 (a slow-rate instruction), and no backpointer
     // row.
+    constexpr int NP = kPreUnits<K, T>, PB = kPrioBase<K, T>;
+    static_assert(NP <= G::C, "the units done ahead are the first chunk's groups");
+    // index of step i's target in the sequence rolled right by `roll`
+    auto target = [&](int i) { return (i - roll < 0) ? i - roll + xlen : i - roll; };
+    // Squares of the first NP units for the target xnext of the coming step
+    // (see kPreUnits).
+    float xnext = 0.0f, pre[NP > 0 ? NP * NCHK : 1];
+    auto presquare = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int un = 0; un < NP; ++un) {
+            float* p = pre + un * NCHK;
+#pragma unroll
+            for (int w = 0; w < NCHK; ++w) p[w] = fsub(un * G::W + w, -xnext);
+#pragma unroll
+            for (int w = 0; w < NCHK; ++w) p[w] = p[w] * p[w];
+#pragma unroll
+            for (int w = 0; w < NCHK; ++w) asm volatile("" : "+v"(p[w]));
+        }
+    };
+    if constexpr (NP > 0) {
+        xnext = xs[0][target(0)];
+        presquare();
+    }
     auto step = [&](auto keys_c, int i) __attribute__((always_inline)) {
         constexpr bool KEYS = decltype(keys_c)::value;
         typedef typename RunType<KEYS>::type run_t;
         constexpr int NCH = KEYS ? kChunkW<K, T> : kChunkWMin<K, T>;  // candidates per chunk
         constexpr int NCHUNK = G::W / NCH;
-        // Target of step i of the sequence rolled right by `roll`.
-        const int u = (i - roll < 0) ? i - roll + xlen : i - roll;
+        const int u = target(i);
 #pragma unroll 1
         for (int tt = 0; tt < ntile; ++tt) {
             // Keep the codebook registers opaque per sequence-step so that
@@ -406,8 +446,23 @@ __device__ __forceinline__ void fwd_run(
                 rp = bslot<K>(ab + wb * G::Q) - (ab + wb * G::Q);
             }
             const int q = q0 + tt;
-            const float negx = -__int_as_float(
-                __builtin_amdgcn_readfirstlane(__float_as_int(xs[tt][u])));
+            // The target: in a VGPR at T = 1, where v_sub_f32 with an SGPR
+            // operand issues at the slow rate (4.25 against 2.5 cycles a
+            // wave64 instruction) and the column chain is 1-3 % faster
+            // (K = 2..7 349k/356k/388k/376k/370k/356k -> 354k/367k/393k/
+            // 385k/380k/367k tiles/s); with several sequences the SGPR form
+            // is as fast (K = 4, 5) or 1 % faster (K = 3, 6, 7), and the
+            // VGPR is better spent.
+            float negx;
+            if constexpr (NP > 0) {
+                negx = -xnext;
+                xnext = xs[0][i + 1 < nsteps ? target(i + 1) : 0];
+            } else if constexpr (T == 1) {
+                negx = -xs[tt][u];
+            } else {
+                negx = -__int_as_float(
+                    __builtin_amdgcn_readfirstlane(__float_as_int(xs[tt][u])));
+            }
             if constexpr (K == 2) __builtin_amdgcn_s_setprio(1);
             const float* bcur = bbuf[tt][i & 1];
 
@@ -445,12 +500,16 @@ __device__ __forceinline__ void fwd_run(
                                            : K == 4 && T == 4 ? U * 7 / 8
                                            : K == 3           ? U * 5 / 8
                                                               : U * 3 / 4;
-                        if (pos == D1) __builtin_amdgcn_s_setprio(1);
-                        if (pos == D0) __builtin_amdgcn_s_setprio(0);
+                        if (pos == D1) __builtin_amdgcn_s_setprio(PB + 1);
+                        if (pos == D0) __builtin_amdgcn_s_setprio(PB);
                     }
                     // candidate costs fl(fl(fl(f - x)^2) + b)
                     float dv[NCH];
-                    if constexpr (KEYS ? kGroupOps<K, T> : kGroupOpsMin<K, T>) {
+                    if (qc * G::C + c < NP) {
+                        // squared at the end of the previous step
+#pragma unroll
+                        for (int w = 0; w < NCH; ++w) dv[w] = pre[c * NCHK + w] + B[blk][w];
+                    } else if constexpr (KEYS ? kGroupOps<K, T> : kGroupOpsMin<K, T>) {
                         // Issue the chunk's candidates opcode by opcode (all
                         // subs, then all squares, then all adds): gfx950
                         // issues adjacent independent v_mul_f32 / v_add_f32
@@ -470,7 +529,7 @@ __device__ __forceinline__ void fwd_run(
 #pragma unroll
                         for (int w = 0; w < NCH; ++w) dv[w] = dv[w] + B[blk][w];
                     } else {
-                        // K <= 3, and K = 4, 5 at T = 1: the compiler's own
+                        // K = 2, and K = 3 at T = 2: the compiler's own
                         // interleaving measures faster.
 #pragma unroll
                         for (int w = 0; w < NCH; ++w) {
@@ -632,11 +691,15 @@ __device__ __forceinline__ void fwd_run(
                 }
             }
         }
+        if constexpr (NP > 0) {
+            __builtin_amdgcn_s_setprio(0);
+            presquare();
+        }
         // The cost stores above are inline ds_write2_b32 the compiler does
         // not track: complete them before the barrier publishes b_{i+1}.
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __syncthreads();
-        __builtin_amdgcn_s_setprio(kPrioTop<K>);
+        __builtin_amdgcn_s_setprio(PB + kPrioTop<K>);
     };
 
     // Min-only steps 0 .. npre-1 (never the last step, which takes the

@@ -123,6 +123,28 @@ def test_short_runs_vs_oracle(hb, oracle_mod, mul1_lut, K):
 
 
 # the deferred-argmin paths ("d*") exist for K >= 4 only
+@pytest.mark.parametrize("K", (3, 4, 5))
+def test_one_sequence_short_runs(hb, oracle_mod, mul1_lut, K, monkeypatch):
+    """One sequence per workgroup squares the next step's first candidates
+    ahead of the barrier: runs of one step (no next target), two, three, and
+    a whole sequence less one, free and pinned, and with the links kept from
+    the middle and the last step only."""
+    monkeypatch.setenv("XTQ_VIT_GROUP", "1")
+    rng = np.random.default_rng(300 + K)
+    for T in (1, 2, 3, 255):
+        X = rng.standard_normal((3, T)).astype(np.float32)
+        X[1] = mul1_lut[rng.integers(0, 65536, T)]
+        ov = rng.integers(0, 1 << (16 - K), 3).astype(np.int32)
+        Xd = torch.from_numpy(X).cuda()
+        for o in (None, ov):
+            for bf in (None, T // 2, T - 1):
+                got = hb.viterbi(Xd, K, back_from=bf,
+                                 overlap=None if o is None else torch.from_numpy(o).cuda())
+                want = oracle_mod.viterbi(X, mul1_lut, K, 16, overlap=o, back_from=bf)
+                np.testing.assert_array_equal(got.cpu().numpy(), want,
+                                              err_msg=f"K={K} T={T} pinned={o is not None} bf={bf}")
+
+
 @pytest.mark.parametrize("group,K", [(g, K) for g in ("1", "2", "4", "8", "fused")
                                      for K in range(2, 8)]
                          + [(g, K) for g in ("d1", "d2", "d4", "d8") for K in range(4, 8)])
