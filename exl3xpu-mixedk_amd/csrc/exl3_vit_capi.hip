@@ -22,7 +22,10 @@
 
 namespace {
 
-enum Code { kMul1 = 0, k3Inst = 1, kMcg = 2, k1Mad = 3, kNumCodes = 4 };
+enum Code {
+    kMul1 = xtq::kCodeMul1, k3Inst = xtq::kCode3Inst, kMcg = xtq::kCodeMcg, k1Mad = xtq::kCode1Mad,
+    kNumCodes = 4
+};
 
 // --------------------------------------------------------- codebook tables
 // fp16 bits -> double (exact).
@@ -923,6 +926,35 @@ int run_host(const float* X, int nseq, int K, Code code, int margin, int pivot,
     return rc;
 }
 
+// The pack and unpack entries over 32- or 64-bit states.
+template <typename S>
+int pack_entry(const S* d_states, int nt, int K, int16_t* d_trellis, void* stream) {
+    std::lock_guard<std::mutex> lk(g_mu);
+    if (!d_states || !d_trellis) return 12;
+    if (K < 2 || K > 7) return 9;
+    if (nt <= 0) return 6;
+    hipError_t e = xtq::launch_pack(K, d_states, nt, d_trellis, (hipStream_t)stream);
+    if (e != hipSuccess) {
+        fprintf(stderr, "xtq_vit pack: %s\n", hipGetErrorString(e));
+        return 4;
+    }
+    return 0;
+}
+
+template <typename S>
+int unpack_entry(const int16_t* d_trellis, int nt, int K, S* d_states, void* stream) {
+    std::lock_guard<std::mutex> lk(g_mu);
+    if (!d_states || !d_trellis) return 12;
+    if (K < 2 || K > 7) return 9;
+    if (nt <= 0) return 6;
+    hipError_t e = xtq::launch_unpack(K, d_trellis, nt, d_states, (hipStream_t)stream);
+    if (e != hipSuccess) {
+        fprintf(stderr, "xtq_vit unpack: %s\n", hipGetErrorString(e));
+        return 4;
+    }
+    return 0;
+}
+
 }  // namespace
 
 extern "C" {
@@ -1136,8 +1168,8 @@ int xtq_trellis_decode_dev(const int16_t* d_trellis, int tk, int tn, int K, cons
     if (current_device(&dev)) return 1;
     rc = dev_init(dev);
     if (rc) return rc;
-    hipError_t e = xtq::launch_decode(K, d_trellis, tk, tn, g_dev[dev].lut[c], d_out_f32,
-                                      d_out_f16, (hipStream_t)stream);
+    hipError_t e = xtq::launch_decode(K, (int)c, d_trellis, tk, tn, d_out_f32, d_out_f16,
+                                      (hipStream_t)stream);
     if (e != hipSuccess) {
         fprintf(stderr, "xtq_vit decode: %s\n", hipGetErrorString(e));
         return 4;
@@ -1147,30 +1179,22 @@ int xtq_trellis_decode_dev(const int16_t* d_trellis, int tk, int tn, int K, cons
 
 int xtq_trellis_pack_dev(const int32_t* d_states, int nt, int K, int16_t* d_trellis,
                          void* stream) {
-    std::lock_guard<std::mutex> lk(g_mu);
-    if (!d_states || !d_trellis) return 12;
-    if (K < 2 || K > 7) return 9;
-    if (nt <= 0) return 6;
-    hipError_t e = xtq::launch_pack(K, d_states, nt, d_trellis, (hipStream_t)stream);
-    if (e != hipSuccess) {
-        fprintf(stderr, "xtq_vit pack: %s\n", hipGetErrorString(e));
-        return 4;
-    }
-    return 0;
+    return pack_entry(d_states, nt, K, d_trellis, stream);
+}
+
+int xtq_trellis_pack64_dev(const int64_t* d_states, int nt, int K, int16_t* d_trellis,
+                           void* stream) {
+    return pack_entry(d_states, nt, K, d_trellis, stream);
 }
 
 int xtq_trellis_unpack_dev(const int16_t* d_trellis, int nt, int K, int32_t* d_states,
                            void* stream) {
-    std::lock_guard<std::mutex> lk(g_mu);
-    if (!d_states || !d_trellis) return 12;
-    if (K < 2 || K > 7) return 9;
-    if (nt <= 0) return 6;
-    hipError_t e = xtq::launch_unpack(K, d_trellis, nt, d_states, (hipStream_t)stream);
-    if (e != hipSuccess) {
-        fprintf(stderr, "xtq_vit unpack: %s\n", hipGetErrorString(e));
-        return 4;
-    }
-    return 0;
+    return unpack_entry(d_trellis, nt, K, d_states, stream);
+}
+
+int xtq_trellis_unpack64_dev(const int16_t* d_trellis, int nt, int K, int64_t* d_states,
+                             void* stream) {
+    return unpack_entry(d_trellis, nt, K, d_states, stream);
 }
 
 int xtq_had128_left_dev(const float* d_ht, const float* d_in, float* d_out, int rows, int cols,

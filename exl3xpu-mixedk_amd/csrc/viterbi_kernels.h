@@ -19,6 +19,9 @@ constexpr int kSteps = 256;
 // Backpointer slots stored per sequence: steps 1..255 of a pass.
 constexpr int kSlots = kSteps - 1;
 
+// The V=1 codebooks.
+enum CodeId { kCodeMul1 = 0, kCode3Inst = 1, kCodeMcg = 2, kCode1Mad = 3 };
+
 // Bytes of backpointers one sequence writes per step, for K bits per weight.
 size_t bp_step_bytes(int K);
 // Bytes of backpointer scratch one sequence needs for a whole pass.
@@ -93,6 +96,9 @@ hipError_t launch_lfac_quads(const float* L, int k, float* Lq, hipStream_t strea
 // out = blockdiag(ht^T) @ in for in, out [rows][cols] fp32 row-major (rows a
 // multiple of 128, in != out), ht[t][r] the weight of input row t in output
 // row r: each output one fp32 fused multiply-add chain in ascending order.
+// With div_rows [rows] and div_cols [cols] the input is first divided by its
+// row's and then by its column's scale; with mul_rows [rows] the output is
+// multiplied by its row's (NULL: not).
 hipError_t launch_had_left(const float* ht, const float* in, float* out, int rows, int cols,
                            hipStream_t stream);
 
@@ -139,16 +145,17 @@ hipError_t launch_traceback(int K, const void* bp, int nseq, const int32_t* send
                             int32_t* states, int16_t* trellis, bool lanes,
                             hipStream_t stream);
 
-// Trellis decode: int16 [tk][tn][16K] -> [16tk][16tn] (fp32 or fp16 bits).
-hipError_t launch_decode(int K, const int16_t* trellis, int tk, int tn,
-                         const float* lut, float* out_f32,
-                         uint16_t* out_f16, hipStream_t stream);
+// Trellis decode: int16 [tk][tn][16K] -> [16tk][16tn] (fp32 and/or fp16 bits)
+// with the codebook `code` (a CodeId).
+hipError_t launch_decode(int K, int code, const int16_t* trellis, int tk, int tn,
+                         float* out_f32, uint16_t* out_f16, hipStream_t stream);
 
-// Pack / unpack between int32 states [nt][256] and int16 trellis [nt][16K].
-hipError_t launch_pack(int K, const int32_t* states, int nt, int16_t* trellis,
-                       hipStream_t stream);
-hipError_t launch_unpack(int K, const int16_t* trellis, int nt, int32_t* states,
-                         hipStream_t stream);
+// Pack / unpack between states [nt][256] (S: int32_t or int64_t) and int16
+// trellis [nt][16K].
+template <typename S>
+hipError_t launch_pack(int K, const S* states, int nt, int16_t* trellis, hipStream_t stream);
+template <typename S>
+hipError_t launch_unpack(int K, const int16_t* trellis, int nt, S* states, hipStream_t stream);
 
 // p[0..n) = v on `stream` (a kernel, so that it may be captured in a graph).
 hipError_t launch_fill_u32(uint32_t* p, uint32_t n, uint32_t v, hipStream_t stream);

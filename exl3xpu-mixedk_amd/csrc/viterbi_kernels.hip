@@ -1356,7 +1356,7 @@ __global__ void fill_u32_kernel(uint32_t* __restrict__ p, uint32_t n, uint32_t v
     if (i < n) p[i] = v;
 }
 
-// ------------------------------------------------- decode / pack / unpack
+// ------------------------------------------------------- tile layout
 // tensor_core_perm (quantize.py:101-118): element t -> row-major 16x16 index.
 __device__ __forceinline__ int tc_perm(int t) {
     const int g = t >> 3, e = t & 7;
@@ -1364,61 +1364,6 @@ __device__ __forceinline__ int tc_perm(int t) {
     const int rr = (e & 1) + ((e & 2) ? 8 : 0);
     const int cc = (e & 4) ? 8 : 0;
     return (r0 + rr) * 16 + c0 + cc;
-}
-
-// 16-bit circular window of the 256K-bit stream ending at bit (t+1)K - 1.
-template <int K>
-__device__ __forceinline__ uint32_t window_state(const uint32_t* words, int t) {
-    constexpr int NB = 256 * K;
-    int b = t * K + K - 16;
-    if (b < 0) b += NB;
-    uint32_t v = 0;
-#pragma unroll
-    for (int k = 0; k < 16; ++k) {
-        int bb = b + k;
-        if (bb >= NB) bb -= NB;
-        v = (v << 1) | ((words[bb >> 5] >> (31 - (bb & 31))) & 1u);
-    }
-    return v;
-}
-
-template <int K>
-__global__ __launch_bounds__(256) void decode_kernel(
-    const int16_t* __restrict__ trellis, int tn, const float* __restrict__ lut,
-    float* __restrict__ out_f32, uint16_t* __restrict__ out_f16) {
-    __shared__ uint32_t words[8 * K];
-    const int tile = blockIdx.x, t = threadIdx.x;
-    const uint32_t* src = (const uint32_t*)(trellis + (size_t)tile * 16 * K);
-    if (t < 8 * K) words[t] = src[t];  // int16 pair [lo, hi] == little-endian u32
-    __syncthreads();
-    const uint32_t s = window_state<K>(words, t);
-    const int p = tc_perm(t);
-    const int a = tile / tn, b = tile - a * tn;
-    const size_t n = (size_t)tn * 16;
-    const size_t idx = (size_t)(16 * a + (p >> 4)) * n + 16 * b + (p & 15);
-    const float v = lut[s];
-    if (out_f32) out_f32[idx] = v;
-    if (out_f16) out_f16[idx] = __builtin_bit_cast(uint16_t, (_Float16)v);
-}
-
-template <int K>
-__global__ __launch_bounds__(256) void unpack_kernel(const int16_t* __restrict__ trellis,
-                                                     int32_t* __restrict__ states) {
-    __shared__ uint32_t words[8 * K];
-    const int tile = blockIdx.x, t = threadIdx.x;
-    const uint32_t* src = (const uint32_t*)(trellis + (size_t)tile * 16 * K);
-    if (t < 8 * K) words[t] = src[t];
-    __syncthreads();
-    states[(size_t)tile * kSteps + t] = (int32_t)window_state<K>(words, t);
-}
-
-template <int K>
-__global__ __launch_bounds__(64) void pack_kernel(const int32_t* __restrict__ states,
-                                                  int16_t* __restrict__ trellis) {
-    const int tile = blockIdx.x, wd = threadIdx.x;
-    if (wd >= 8 * K) return;
-    store_word(trellis + (size_t)tile * 16 * K + 2 * wd,
-               pack_word<K>(states + (size_t)tile * kSteps, wd));
 }
 
 // ------------------------------------------------- BlockLDLQ column chains
@@ -2060,32 +2005,6 @@ struct TbL {
 };
 
 template <int K>
-struct DecL {
-    static hipError_t run(const int16_t* tr, int tk, int tn, const float* lut,
-                          float* of, uint16_t* oh, hipStream_t s) {
-        hipLaunchKernelGGL(decode_kernel<K>, dim3(tk * tn), dim3(256), 0, s, tr, tn, lut,
-                           of, oh);
-        return hipGetLastError();
-    }
-};
-
-template <int K>
-struct PackL {
-    static hipError_t run(const int32_t* st, int nt, int16_t* tr, hipStream_t s) {
-        hipLaunchKernelGGL(pack_kernel<K>, dim3(nt), dim3(64), 0, s, st, tr);
-        return hipGetLastError();
-    }
-};
-
-template <int K>
-struct UnpackL {
-    static hipError_t run(const int16_t* tr, int nt, int32_t* st, hipStream_t s) {
-        hipLaunchKernelGGL(unpack_kernel<K>, dim3(nt), dim3(256), 0, s, tr, st);
-        return hipGetLastError();
-    }
-};
-
-template <int K>
 struct StepBytes {
     static hipError_t run(size_t* out) {
         *out = (size_t)Geom<K>::BPSTEP;
@@ -2191,24 +2110,6 @@ hipError_t launch_traceback(int K, const void* bp, int nseq, const int32_t* send
         return hipErrorInvalidValue;
     return dispatch_k<TbL>(K, bp, nseq, send, nsteps, stop, shift, sout, states, trellis,
                            lanes, stream);
-}
-
-hipError_t launch_decode(int K, const int16_t* trellis, int tk, int tn, const float* lut,
-                         float* out_f32, uint16_t* out_f16, hipStream_t stream) {
-    if (tk <= 0 || tn <= 0) return hipSuccess;
-    return dispatch_k<DecL>(K, trellis, tk, tn, lut, out_f32, out_f16, stream);
-}
-
-hipError_t launch_pack(int K, const int32_t* states, int nt, int16_t* trellis,
-                       hipStream_t stream) {
-    if (nt <= 0) return hipSuccess;
-    return dispatch_k<PackL>(K, states, nt, trellis, stream);
-}
-
-hipError_t launch_unpack(int K, const int16_t* trellis, int nt, int32_t* states,
-                         hipStream_t stream) {
-    if (nt <= 0) return hipSuccess;
-    return dispatch_k<UnpackL>(K, trellis, nt, states, stream);
 }
 
 size_t defer_tile_bytes(int K) {

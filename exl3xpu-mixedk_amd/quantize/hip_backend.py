@@ -61,7 +61,9 @@ def lib():
         L.xtq_vit_viterbi_dev.argtypes = [vp, i32, i32, i32, cp, vp, i32, vp, vp]
         L.xtq_trellis_decode_dev.argtypes = [vp, i32, i32, i32, cp, vp, vp, vp]
         L.xtq_trellis_pack_dev.argtypes = [vp, i32, i32, vp, vp]
+        L.xtq_trellis_pack64_dev.argtypes = [vp, i32, i32, vp, vp]
         L.xtq_trellis_unpack_dev.argtypes = [vp, i32, i32, vp, vp]
+        L.xtq_trellis_unpack64_dev.argtypes = [vp, i32, i32, vp, vp]
         L.xtq_vit_get_lut.argtypes = [cp, vp]
         L.xtq_had128_left_dev.argtypes = [vp, vp, vp, i32, i32, vp]
         L.xtq_had128_right_dev.argtypes = [vp, vp, vp, i32, i32, vp]
@@ -305,22 +307,21 @@ def pack(states: torch.Tensor, K: int) -> torch.Tensor:
     out = torch.empty(nt, 16 * K, dtype=torch.int16, device=st.device)
     if nt:
         with torch.cuda.device(st.device):
-            rc = lib().xtq_trellis_pack_dev(st.data_ptr(), nt, int(K), out.data_ptr(),
-                                            _stream(st.device))
-        _check("xtq_trellis_pack_dev", rc)
+            rc = getattr(lib(), fn)(st.data_ptr(), nt, int(K), out.data_ptr(),
+                                    _stream(st.device))
+        _check(fn, rc)
     return out
 
 
-def unpack(trellis: torch.Tensor, K: int) -> torch.Tensor:
-    """int16 trellis [nt, 16K] (device) -> int32 states [nt, 256]."""
+def _unpack(trellis: torch.Tensor, K: int, dtype: torch.dtype, fn: str) -> torch.Tensor:
     tr = _dev_tensor(trellis, torch.int16, "trellis").view(-1, 16 * K)
     nt = tr.shape[0]
-    out = torch.empty(nt, 256, dtype=torch.int32, device=tr.device)
+    out = torch.empty(nt, 256, dtype=dtype, device=tr.device)
     if nt:
         with torch.cuda.device(tr.device):
-            rc = lib().xtq_trellis_unpack_dev(tr.data_ptr(), nt, int(K), out.data_ptr(),
-                                              _stream(tr.device))
-        _check("xtq_trellis_unpack_dev", rc)
+            rc = getattr(lib(), fn)(tr.data_ptr(), nt, int(K), out.data_ptr(),
+                                    _stream(tr.device))
+        _check(fn, rc)
     return out
 
 
@@ -349,6 +350,26 @@ def chunk_seqs(nseq: int, K: int):
 def prof_enable(on: bool = True):
     """Bracket every forward/traceback launch with HIP events (benchmarks)."""
     lib().xtq_vit_prof_enable(1 if on else 0)
+
+def pack(states: torch.Tensor, K: int) -> torch.Tensor:
+    """int32 states [nt, 256] (device) -> int16 trellis [nt, 16K]."""
+    return _pack(states, K, torch.int32, "xtq_trellis_pack_dev")
+
+
+def pack64(states: torch.Tensor, K: int) -> torch.Tensor:
+    """int64 states [nt, 256] (device) -> int16 trellis [nt, 16K]."""
+    return _pack(states, K, torch.int64, "xtq_trellis_pack64_dev")
+
+
+def unpack(trellis: torch.Tensor, K: int) -> torch.Tensor:
+    """int16 trellis [nt, 16K] (device) -> int32 states [nt, 256]."""
+    return _unpack(trellis, K, torch.int32, "xtq_trellis_unpack_dev")
+
+
+def unpack64(trellis: torch.Tensor, K: int) -> torch.Tensor:
+    """int16 trellis [nt, 16K] (device) -> int64 states [nt, 256]."""
+    return _unpack(trellis, K, torch.int64, "xtq_trellis_unpack64_dev")
+
 
 
 def prof_read() -> dict:

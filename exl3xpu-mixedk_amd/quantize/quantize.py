@@ -402,16 +402,18 @@ def pack_states(states: torch.Tensor, K: int, V: int = 1) -> torch.Tensor:
     words MSB first, stored as int16 halves, low half first."""
     if V != 1:
         raise NotImplementedError("V=1 only")
-    st = _on_gpu(states).to(torch.int32).reshape(-1, 256)
-    return _hb.pack(st, K).to(states.device)
+    st = _on_gpu(states)
+    if st.dtype == torch.int64:              # read as they are: no int32 copy
+        return _hb.pack64(st.reshape(-1, 256), K).to(states.device)
+    return _hb.pack(st.to(torch.int32).reshape(-1, 256), K).to(states.device)
 
 
 def unpack_states(trellis: torch.Tensor, K: int, V: int = 1) -> torch.Tensor:
     """int16 [..., 16K] -> states [..., 256] int64 (quantize.py:381-402)."""
     if V != 1:
         raise NotImplementedError("V=1 only")
-    st = _hb.unpack(_on_gpu(trellis).reshape(-1, 16 * K), K)
-    return st.long().view(*trellis.shape[:-1], 256).to(trellis.device)
+    st = _hb.unpack64(_on_gpu(trellis).reshape(-1, 16 * K), K)
+    return st.view(*trellis.shape[:-1], 256).to(trellis.device)
 
 
 def decode_trellis(trellis: torch.Tensor, lut: torch.Tensor, K: int, k: int, n: int,

@@ -255,6 +255,12 @@ XTQ_API int xtq_trellis_pack_dev(const int32_t* d_states, int nt, int K, int16_t
                          void* stream);
 XTQ_API int xtq_trellis_unpack_dev(const int16_t* d_trellis, int nt, int K, int32_t* d_states,
                            void* stream);
+/* The same over int64 states, as the host API (and the reference) holds them:
+ * no conversion pass over the states on either side. */
+XTQ_API int xtq_trellis_pack64_dev(const int64_t* d_states, int nt, int K, int16_t* d_trellis,
+                           void* stream);
+XTQ_API int xtq_trellis_unpack64_dev(const int16_t* d_trellis, int nt, int K, int64_t* d_states,
+                           void* stream);
 
 /*
  * Device-pointer block-128 transform on the first dimension: the HIP
