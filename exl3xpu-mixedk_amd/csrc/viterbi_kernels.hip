@@ -1509,86 +1509,6 @@ __global__ __launch_bounds__(256) void lfac_quads_kernel(const float* __restrict
     }
 }
 
-// ------------------------------------------------- block-128 Hadamard
-// out[128b + r][c] = sum_{t=0..127} ht[t][r] * in[128b + t][c] (had_left,
-// quantize.py:134-138, with ht = h^T: the multipliers by input row),
-// evaluated as torch's CPU sgemm evaluates it: one fp32 fused multiply-add
-// chain per output over t ascending, from zero (measured bit for bit against
-// an fmaf chain).  Taking h^T makes the 16 multipliers a wave needs at step t
-// one contiguous, wave-uniform row segment (scalar loads).  Wave: 16 rows x
-// 64 columns; workgroup: 4 waves.
-__global__ __launch_bounds__(256) void had_left_kernel(const float* __restrict__ ht,
-                                                       const float* __restrict__ in,
-                                                       float* __restrict__ out, int cols) {
-    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ln = threadIdx.x & 63;
-    const int c = blockIdx.x * 64 + ln;
-    const int r0 = (blockIdx.z * 4 + wv) * 16;
-    const bool live = c < cols;
-    const float* src = in + (size_t)blockIdx.y * 128 * cols + (live ? c : 0);
-    float acc[16];
-#pragma unroll
-    for (int q = 0; q < 16; ++q) acc[q] = 0.0f;
-    for (int t = 0; t < 128; ++t) {
-        const float w = src[(size_t)t * cols];
-        const float* hr = ht + t * 128 + r0;
-#pragma unroll
-        for (int q = 0; q < 16; ++q) acc[q] = __builtin_fmaf(hr[q], w, acc[q]);
-    }
-    if (live) {
-        float* dst = out + ((size_t)blockIdx.y * 128 + r0) * cols + c;
-#pragma unroll
-        for (int q = 0; q < 16; ++q) dst[(size_t)q * cols] = acc[q];
-    }
-}
-
-// out[r][128b + c] = sum_{t=0..127} h[t][c] * in[r][128b + t] (had_right,
-// quantize.py:141-145) without a transpose: each output one fp32 fused
-// multiply-add chain over t ascending, from zero -- the products and the
-// order of had_left_kernel on the transpose, hence torch's CPU sgemm bits.
-// Wave: 8 rows x 64 columns (half of a 128-column block); the 8 inputs of a
-// step t are wave-uniform (scalar loads, 8 consecutive t per row at a time)
-// and the multipliers h[t][c] one coalesced row segment.  Workgroup: 4
-// waves, 32 rows.  (16 rows per wave with 4 steps per scalar load measured
-// 1.7x slower: twice the scalar loads per multiply-add.)
-constexpr int kHrRows = 8;                 // rows per wave
-constexpr int kHrT = 8;                    // steps per scalar load
-__global__ __launch_bounds__(256) void had_right_kernel(const float* __restrict__ h,
-                                                        const float* __restrict__ in,
-                                                        float* __restrict__ out, int rows,
-                                                        int cols) {
-    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ln = threadIdx.x & 63;
-    const int b = blockIdx.x >> 1;                          // 128-column block
-    const int c = ((blockIdx.x & 1) << 6) + ln;             // column within the block
-    const int r0 = (blockIdx.y * 4 + wv) * kHrRows;
-    if (r0 >= rows) return;
-    const int nr = rows - r0 < kHrRows ? rows - r0 : kHrRows;   // wave-uniform
-    const float* src = in + (size_t)r0 * cols + 128 * b;
-    float acc[kHrRows];
-#pragma unroll
-    for (int q = 0; q < kHrRows; ++q) acc[q] = 0.0f;
-    if (nr == kHrRows) {
-        for (int t0 = 0; t0 < 128; t0 += kHrT) {
-#pragma unroll
-            for (int t = t0; t < t0 + kHrT; ++t) {
-                const float hv = h[t * 128 + c];
-#pragma unroll
-                for (int q = 0; q < kHrRows; ++q)
-                    acc[q] = __builtin_fmaf(hv, src[(size_t)q * cols + t], acc[q]);
-            }
-        }
-    } else {
-        for (int t = 0; t < 128; ++t) {
-            const float hv = h[t * 128 + c];
-            for (int q = 0; q < nr; ++q)
-                acc[q] = __builtin_fmaf(hv, src[(size_t)q * cols + t], acc[q]);
-        }
-    }
-    float* dst = out + (size_t)r0 * cols + 128 * b + c;
-#pragma unroll
-    for (int q = 0; q < kHrRows; ++q)
-        if (q < nr) dst[(size_t)q * cols] = acc[q];
-}
-
 template <int K>
 __global__ __launch_bounds__(kFwdThreads) void ldlq_chain_kernel(
     const float* __restrict__ W, const float* __restrict__ Lq, int k, int n, int jc0, int tnl,
@@ -2056,26 +1976,6 @@ hipError_t launch_tailbite_fused(int K, const float* X, int nseq, const float* l
         return hipErrorInvalidValue;
     return dispatch_k<FusedL>(K, X, nseq, lut, pivot, n1, bp, send, ovbuf, flags, counter,
                               epoch, spin_limit, err, stream);
-}
-
-hipError_t launch_had_left(const float* ht, const float* in, float* out, int rows, int cols,
-                           hipStream_t stream) {
-    if (rows <= 0 || cols <= 0) return hipSuccess;
-    if (rows % 128 || rows / 128 > 65535) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(had_left_kernel, dim3((cols + 63) / 64, rows / 128, 2), dim3(256), 0,
-                       stream, ht, in, out, cols);
-    return hipGetLastError();
-}
-
-hipError_t launch_had_right(const float* h, const float* in, float* out, int rows, int cols,
-                            hipStream_t stream) {
-    if (rows <= 0 || cols <= 0) return hipSuccess;
-    if (cols % 128) return hipErrorInvalidValue;
-    const int ry = (rows + 4 * kHrRows - 1) / (4 * kHrRows);
-    if (ry > 65535) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(had_right_kernel, dim3(cols / 64, ry), dim3(256), 0, stream, h, in, out,
-                       rows, cols);
-    return hipGetLastError();
 }
 
 hipError_t launch_lfac_quads(const float* L, int k, float* Lq, hipStream_t stream) {

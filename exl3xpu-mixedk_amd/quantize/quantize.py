@@ -169,9 +169,23 @@ def had_right(w: torch.Tensor, h: torch.Tensor) -> torch.Tensor:
     return torch.matmul(w.view(k, n // 128, 128), h).view(k, n)
 
 
+def _fold_scales(w: torch.Tensor, suh: torch.Tensor, svh: torch.Tensor) -> bool:
+    """Whether the kernels apply the channel scales in the transforms' passes:
+    fp32 GPU weights with one scale per row and per column there.  Anything
+    else takes the separate torch passes below."""
+    return (w.is_cuda and w.dtype == torch.float32 and w.dim() == 2
+            and w.shape[0] % 128 == 0 and w.shape[1] % 128 == 0
+            and suh.shape == w.shape[:1] and svh.shape == w.shape[1:]
+            and suh.device == w.device and svh.device == w.device)
+
+
 def to_inner(w_orig: torch.Tensor, suh: torch.Tensor, svh: torch.Tensor,
              h: torch.Tensor) -> torch.Tensor:
     """W_orig [k, n] -> W_inner = B_k diag(1/suh) W diag(1/svh) B_n."""
+    if _fold_scales(w_orig, suh, svh):
+        hd = h.to(w_orig.device, torch.float32)
+        w = _hb.had128_left(w_orig.contiguous(), hd, div_rows=suh.float(), div_cols=svh.float())
+        return _hb.had128_right(w, hd)
     w = w_orig / suh.float().unsqueeze(1)
     w = w / svh.float().unsqueeze(0)
     return had_right(had_left(w, h), h)
@@ -180,6 +194,10 @@ def to_inner(w_orig: torch.Tensor, suh: torch.Tensor, svh: torch.Tensor,
 def from_inner(w_inner: torch.Tensor, suh: torch.Tensor, svh: torch.Tensor,
                h: torch.Tensor) -> torch.Tensor:
     """W_inner -> W_orig = diag(suh) B_k W_i B_n diag(svh)."""
+    if _fold_scales(w_inner, suh, svh):
+        hd = h.to(w_inner.device, torch.float32)
+        w = _hb.had128_left(w_inner.contiguous(), hd, mul_rows=suh.float())
+        return _hb.had128_right(w, hd, mul_cols=svh.float())
     w = had_left(w_inner, h) * suh.float().unsqueeze(1)
     return had_right(w, h) * svh.float().unsqueeze(0)
 

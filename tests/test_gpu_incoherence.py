@@ -1,0 +1,45 @@
+"""The block-128 transforms with the channel scales folded into their passes
+against the same arithmetic on the CPU (torch's sgemm sums every output as one
+fp32 multiply-add chain in ascending order), bit for bit."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def xq():
+    import quantize
+    assert torch.cuda.is_available(), "GPU tests need a HIP device"
+    return quantize
+
+
+@pytest.mark.parametrize("k,n", [(128, 128), (256, 128), (128, 384), (640, 1152)])
+def test_scaled_transforms_match_cpu(xq, k, n):
+    """to_inner and from_inner with magnitudes whose quotients round, and the
+    forms that keep their separate passes: a transposed view, fp64 scales."""
+    g = torch.Generator().manual_seed(k + n)
+    w = torch.randn(k, n, generator=g)
+    su = (torch.randn(k, generator=g).abs() + 0.1).half()
+    sv = (torch.randn(n, generator=g) + 3.0).half()
+    h = xq.hadamard128(None, torch.float32)
+    want_in = xq.to_inner(w, su, sv, h)
+    want_out = xq.from_inner(w, su, sv, h)
+    sud, svd, hd = su.cuda(), sv.cuda(), h.cuda()
+    for wd in (w.cuda(), w.t().contiguous().cuda().t()):
+        assert torch.equal(xq.to_inner(wd, sud, svd, hd).cpu(), want_in)
+        assert torch.equal(xq.from_inner(wd, sud, svd, hd).cpu(), want_out)
+    assert torch.equal(xq.to_inner(w.cuda(), sud.double(), svd.double(), hd).cpu(), want_in)
+
+
+@pytest.mark.parametrize("cols", (1, 63, 64, 65, 200))
+def test_had_left_ragged_columns(xq, cols):
+    """Column counts around the kernel's 64-column tiles, and more tiles than
+    workgroups of one launch."""
+    rows = 128 * (600 if cols == 1 else 2)
+    w = torch.randn(rows, cols, generator=torch.Generator().manual_seed(cols))
+    h = xq.hadamard128(None, torch.float32)
+    # the CPU product of the padded matrix: torch sums narrow ones otherwise
+    pad = torch.cat([w, torch.zeros(rows, 256 - cols)], 1)
+    want = xq.had_left(pad, h)[:, :cols]
+    assert torch.equal(xq.had_left(w.cuda(), h.cuda()).cpu(), want)
