@@ -538,16 +538,10 @@ int tailbite_chunks(DevCtx& cx, const TbScratch& w, int chunk, const float* dX, 
         }
         if (use_fused(cx, n)) {
             if (++cx.epoch == 0) cx.epoch = 1;
-            int pf = pbeg(0, (double)n * (n1 + xtq::kSteps));
-            e = xtq::launch_tailbite_fused(K, x, n, lut, pivot, n1, w.bp, w.send, w.ov, w.flags,
-                                           w.counter, cx.epoch, kSpinLimit, w.err, s);
+            const int pf = pbeg(0, (double)n * (n1 + xtq::kSteps));
+            e = xtq::launch_tailbite_fused(K, x, n, lut, pivot, n1, w.bp, w.ov, w.flags,
+                                           w.counter, cx.epoch, kSpinLimit, w.err, st, tr, s);
             prof_end(pf, s);
-            if (e == hipSuccess) {
-                pf = pbeg(1, 0.0);
-                e = xtq::launch_traceback(K, w.bp, n, w.send, xtq::kSteps, 0, 0, nullptr, st,
-                                          tr, use_lanes(n), s);
-                prof_end(pf, s);
-            }
             if (e != hipSuccess) {
                 fprintf(stderr, "xtq_vit run: %s\n", hipGetErrorString(e));
                 return 4;

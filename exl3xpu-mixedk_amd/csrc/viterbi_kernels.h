@@ -77,16 +77,17 @@ hipError_t launch_traceback_defer(int K, const void* bm, const float* X, int xst
 // Both tail-biting passes of nseq sequences (256-step targets X [nseq][256])
 // in one launch of 2*nseq workgroups (see tailbite_fused_kernel): pass 1
 // free on X rolled by pivot for n1 steps, traced back in-kernel to
-// ov = s_pivot >> K (ovbuf), pass 2 pinned to ov; send receives the pass-2
-// final states and bp the pass-2 backpointers (trace them back with
-// launch_traceback(K, bp, nseq, send, 256, 0, ...)).  flags [nseq] must hold
-// values != epoch on entry (epoch increases per launch; zero-filled memory
-// and epoch >= 1 work); counter is one device word.  err |= 2 when a pass-2
-// wait expires after spin_limit polls, |= 4 on a task outside the launch.
+// ov = s_pivot >> K (ovbuf), pass 2 pinned to ov and traced back to the
+// states [nseq][256] and/or the packed trellis [nseq][16K] (each nullable).
+// flags [nseq] must hold values != epoch on entry (epoch increases per
+// launch; zero-filled memory and epoch >= 1 work); counter is one device
+// word.  err |= 2 when a pass-2 wait expires after spin_limit polls, |= 4 on a
+// task outside the launch.
 hipError_t launch_tailbite_fused(int K, const float* X, int nseq, const float* lut,
-                                 int pivot, int n1, void* bp, int32_t* send, int32_t* ovbuf,
-                                 uint32_t* flags, int32_t* counter, uint32_t epoch,
-                                 int spin_limit, uint32_t* err, hipStream_t stream);
+                                 int pivot, int n1, void* bp, int32_t* ovbuf, uint32_t* flags,
+                                 int32_t* counter, uint32_t epoch, int spin_limit,
+                                 uint32_t* err, int32_t* states, int16_t* trellis,
+                                 hipStream_t stream);
 
 // Writes the block-LDL factor L [k][k] (row-major, k a multiple of 16) into
 // Lq (k*k floats) in the chain feedback's quad layout (see

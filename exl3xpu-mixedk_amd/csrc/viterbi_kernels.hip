@@ -1285,16 +1285,24 @@ __global__ __launch_bounds__(kTbLaneSeqs) void tb_defer_kernel(
 // so that an unexpected stall ends the launch with an error instead of a
 // hang.  With n = 320 on 256 CUs the 640 passes fill 3 rounds instead of the
 // 4 of two separate launches.  Pass-2 backpointers reuse the sequence's
-// pass-1 slots (pass 1 has finished reading them before it publishes); the
-// pass-2 traceback runs as tb_kernel afterwards.
+// pass-1 slots (pass 1 has finished reading them before it publishes) and are
+// traced back in the same workgroup, which writes the states and the packed
+// trellis: the 1024-thread chase with its loads two chunks ahead
+// (tb_chase_pf) takes 20-30 us where a tb_kernel launch after the passes took
+// 86 (64 tiles, K=2) to 108 us (1003 tiles, K=5) and its gap.
 template <int K>
 __global__ __launch_bounds__(kFwdThreads) void tailbite_fused_kernel(
     const float* __restrict__ X, int nseq, const float* __restrict__ lut, int pivot,
-    int n1, uint8_t* __restrict__ bp, int32_t* __restrict__ send, int32_t* __restrict__ ovbuf,
-    uint32_t* __restrict__ flags, int32_t* __restrict__ counter, uint32_t epoch,
-    int spin_limit, uint32_t* __restrict__ err) {
+    int n1, uint8_t* __restrict__ bp, int32_t* __restrict__ ovbuf, uint32_t* __restrict__ flags,
+    int32_t* __restrict__ counter, uint32_t epoch, int spin_limit, uint32_t* __restrict__ err,
+    int32_t* __restrict__ states, int16_t* __restrict__ trellis) {
     using G = Geom<K>;
     __shared__ FwdSmem<K, 1> sm;
+    // traceback staging: the forward's b buffers where they hold 64 KiB
+    constexpr bool kOwnStage = 2 * sizeof(float) * G::SPL < (size_t)kTbStage;
+    __shared__ __attribute__((aligned(16))) uint4 tbstage[kOwnStage ? kTbStage / 16 : 1];
+    uint4* const stage = kOwnStage ? tbstage : (uint4*)&sm.bbuf[0][0][0];
+    __shared__ int32_t st[kSteps];
     __shared__ int32_t task, cur;
     const int tid = threadIdx.x;
     if (tid == 0) task = atomicAdd(counter, 1);
@@ -1313,9 +1321,8 @@ __global__ __launch_bounds__(kFwdThreads) void tailbite_fused_kernel(
         // overwrite them) before any thread reads them back.
         __threadfence();
         __syncthreads();
-        const uint8_t* bpq = bp + (size_t)t * ((size_t)kSlots * G::BPSTEP);
-        tb_chase<K>(bpq, n1, pivot, (uint4*)&sm.bbuf[0][0][0], (int)sizeof(sm.bbuf), nullptr,
-                    cur);
+        tb_chase_pf<K>(bp + (size_t)t * ((size_t)kSlots * G::BPSTEP), n1, pivot, stage, nullptr,
+                       cur);
         if (tid == 0) {
             __hip_atomic_store(&ovbuf[t], cur >> K, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             __hip_atomic_store(&flags[t], epoch, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
@@ -1340,8 +1347,19 @@ __global__ __launch_bounds__(kFwdThreads) void tailbite_fused_kernel(
         }
         __syncthreads();
         if (sm.ovs[0] < 0) return;             // wait expired: reported through err
-        fwd_run<K, 1>(sm, X, kSteps, kSteps, q, 1, lut, 0, kSteps, 0, true, bp, send + q,
-                      err, tid);
+        fwd_run<K, 1>(sm, X, kSteps, kSteps, q, 1, lut, 0, kSteps, 0, true, bp, &cur, err, tid);
+        // the rows are read back by the workgroup that wrote them: the
+        // barrier's workgroup-scope ordering suffices (as in the column chain)
+        __syncthreads();
+        if (tid == 0) st[kSteps - 1] = cur & 0xFFFF;
+        __syncthreads();
+        tb_chase_pf<K>(bp + (size_t)q * ((size_t)kSlots * G::BPSTEP), kSteps, 0, stage, st, cur);
+        if (tid < kSteps) {
+            if (states) states[(size_t)q * kSteps + tid] = st[tid];
+        } else if (trellis && tid < kSteps + 8 * K) {
+            const int wd = tid - kSteps;
+            store_word(trellis + (size_t)q * 16 * K + 2 * wd, pack_word<K>(st, wd));
+        }
     }
 }
 
@@ -1880,13 +1898,13 @@ struct DeferBytes {
 template <int K>
 struct FusedL {
     static hipError_t run(const float* X, int nseq, const float* lut, int pivot, int n1,
-                          void* bp, int32_t* send, int32_t* ovbuf, uint32_t* flags,
-                          int32_t* counter, uint32_t epoch, int spin_limit, uint32_t* err,
-                          hipStream_t s) {
+                          void* bp, int32_t* ovbuf, uint32_t* flags, int32_t* counter,
+                          uint32_t epoch, int spin_limit, uint32_t* err, int32_t* states,
+                          int16_t* trellis, hipStream_t s) {
         hipLaunchKernelGGL(reset_counter_kernel, dim3(1), dim3(1), 0, s, counter);
         hipLaunchKernelGGL(tailbite_fused_kernel<K>, dim3(2 * nseq), dim3(kFwdThreads), 0, s,
-                           X, nseq, lut, pivot, n1, (uint8_t*)bp, send, ovbuf, flags,
-                           counter, epoch, spin_limit, err);
+                           X, nseq, lut, pivot, n1, (uint8_t*)bp, ovbuf, flags, counter, epoch,
+                           spin_limit, err, states, trellis);
         return hipGetLastError();
     }
 };
@@ -1968,14 +1986,15 @@ hipError_t launch_forward(int K, const float* X, int xstride, int xlen, int nseq
 }
 
 hipError_t launch_tailbite_fused(int K, const float* X, int nseq, const float* lut,
-                                 int pivot, int n1, void* bp, int32_t* send, int32_t* ovbuf,
-                                 uint32_t* flags, int32_t* counter, uint32_t epoch,
-                                 int spin_limit, uint32_t* err, hipStream_t stream) {
+                                 int pivot, int n1, void* bp, int32_t* ovbuf, uint32_t* flags,
+                                 int32_t* counter, uint32_t epoch, int spin_limit,
+                                 uint32_t* err, int32_t* states, int16_t* trellis,
+                                 hipStream_t stream) {
     if (nseq <= 0) return hipSuccess;
     if (pivot < 0 || pivot >= kSteps || n1 <= pivot || n1 > kSteps || spin_limit < 1)
         return hipErrorInvalidValue;
-    return dispatch_k<FusedL>(K, X, nseq, lut, pivot, n1, bp, send, ovbuf, flags, counter,
-                              epoch, spin_limit, err, stream);
+    return dispatch_k<FusedL>(K, X, nseq, lut, pivot, n1, bp, ovbuf, flags, counter, epoch,
+                              spin_limit, err, states, trellis, stream);
 }
 
 hipError_t launch_lfac_quads(const float* L, int k, float* Lq, hipStream_t stream) {
