@@ -419,7 +419,7 @@ int pick_group(const DevCtx& cx, int K, int n) {
         // Test hook: force the sequences per workgroup (1, 2, 4 or 8), clamped
         // to what the LDS footprint for K allows.
         const int want = atoi(g);
-        const int cap = xtq::forward_group(K, 1 << 30, 1);
+        const int cap = xtq::forward_group_max(K);
         if (want == 1 || want == 2 || want == 4 || want == 8) T = want < cap ? want : cap;
     }
     return T;
@@ -437,15 +437,51 @@ int scratch_end(DevCtx& cx, hipStream_t s, bool sync) {
     return sync ? finish(cx, s) : 0;
 }
 
+// Steps until the last of a fused launch's 2n workgroups ends: each CU takes
+// the next of n first passes and then of n second passes, of d1 and d2 steps,
+// as soon as it is free.
+double fused_steps(int n, int d1, int d2, int ncu) {
+    const int r = n / ncu, m = n % ncu;        // pass 1: m CUs take r + 1, the others r
+    const int cus[2] = {ncu - m, m};
+    double t[2] = {(double)r * d1, (double)(r + 1) * d1};
+    double end = m ? t[1] : t[0];
+    for (int left = n; left > 0;) {
+        const int g = m && t[1] < t[0] ? 1 : 0;            // the CUs free first
+        t[g] = (t[g] < d1 ? d1 : t[g]) + d2;               // (a pass 2 waits for its pass 1)
+        if (t[g] > end) end = t[g];
+        left -= cus[g];
+    }
+    return end;
+}
+
 // Whether a chunk of n sequences runs as one fused two-pass launch:
-// XTQ_VIT_FUSED=0 never, =1 always, unset: batches below 4 sequences per CU
-// (where separate pass launches leave CUs idle in their last round).
-bool use_fused(const DevCtx& cx, int n) {
+// XTQ_VIT_FUSED=0 never, =1 always, unset: if it is estimated to end before
+// the separate launches (with XTQ_VIT_GROUP set: below 4 sequences per CU, as
+// a group asks for separate launches above).  The fused launch runs one
+// sequence per workgroup, traces back inside (the time of about 7 and 16
+// steps; at K=2, whose rows are 4 KiB, 24 and 48) and fills its rounds with 2n
+// passes; separate launches run T sequences per
+// workgroup (1.17 against 1.33 us per step and sequence at K=4) and read all
+// backpointer rows again, at 4.7 TB/s up to the 0.3 ms that one-lane
+// tracebacks take at any size.  Measured, fused / separate, ms: K=4 320 tiles
+// 1.07 / 1.36, 512 1.42 / 1.39, 768 2.09 / 2.21, 1003 2.78 / 2.53, 1100 3.10 /
+// 3.69, 2100 5.91 / 7.67; K=7 1003 3.00 / 2.67; K=2 3700 11.8 / 11.0.
+bool use_fused(const DevCtx& cx, int K, int n, int n1) {
     if (const char* e = getenv("XTQ_VIT_FUSED")) {
         if (!strcmp(e, "0")) return false;
         if (!strcmp(e, "1")) return true;
     }
-    return n < 4 * (cx.ncu > 0 ? cx.ncu : 1);
+    const int ncu = cx.ncu > 0 ? cx.ncu : 1;
+    if (getenv("XTQ_VIT_GROUP")) return n < 4 * ncu;
+    // (beyond, a round is a small part of the whole and T decides)
+    if (n >= 16 * ncu) return false;
+    double rows = 1.5e-6 / 4.7 * (double)xtq::bp_tile_bytes(K) * n;      // us
+    if (rows > 300.0) rows = 300.0;
+    const double split =
+        xtq::forward_cost_us(K, xtq::forward_group(K, n, ncu), n, ncu) * (n1 + xtq::kSteps);
+    const int tb1 = K == 2 ? 24 : 7, tb2 = K == 2 ? 48 : 16;     // steps' time per traceback
+    return fused_steps(n, n1 + tb1, xtq::kSteps + tb2, ncu) * xtq::forward_step_us(K, 1) <=
+           split + rows + 50.0;
 }
 
 // Whether the tracebacks of a chunk of n sequences use one lane per
@@ -536,7 +572,7 @@ int tailbite_chunks(DevCtx& cx, const TbScratch& w, int chunk, const float* dX, 
             }
             continue;
         }
-        if (use_fused(cx, n)) {
+        if (use_fused(cx, K, n, n1)) {
             if (++cx.epoch == 0) cx.epoch = 1;
             const int pf = pbeg(0, (double)n * (n1 + xtq::kSteps));
             e = xtq::launch_tailbite_fused(K, x, n, lut, pivot, n1, w.bp, w.ov, w.flags,

@@ -64,7 +64,7 @@
  *                    (0: always, -1: never; default 2048)
  *   XTQ_VIT_FUSED    0: always run the two tail-biting passes as separate
  *                    launches; 1: always as one fused launch (testing);
- *                    default: fused for batches under 4 sequences per CU
+ *                    default: whichever is estimated to end first
  */
 #ifndef EXL3_VIT_H
 #define EXL3_VIT_H

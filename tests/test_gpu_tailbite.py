@@ -535,3 +535,20 @@ def test_verify_viterbi_readme_case(hb, oracle_mod, mul1_lut):
     mse_r = float(((mul1_lut[ref] - X) ** 2).mean())
     assert mse_k == mse_r
     assert int(((out[:, 0] >> 4) == (out[:, -1] & ((1 << 12) - 1))).sum()) == nseq
+
+
+@pytest.mark.parametrize("K", range(2, 8))
+def test_batch_route_edges(hb, K, monkeypatch):
+    """Batch sizes on both sides of the route rules (fused or separate passes,
+    sequences per workgroup): the default route's states and trellis equal
+    the one-sequence separate launches'."""
+    g = torch.Generator().manual_seed(70 + K)
+    X = torch.randn(2049, 256, generator=g).cuda()
+    for n in (255, 257, 511, 512, 513, 769, 1003, 1023, 1024, 1537, 2049):
+        for name in ("XTQ_VIT_FUSED", "XTQ_VIT_GROUP"):
+            monkeypatch.delenv(name, raising=False)
+        st, tr = hb.tailbite(X[:n], K, 147, 16, trellis=True)
+        monkeypatch.setenv("XTQ_VIT_FUSED", "0")
+        monkeypatch.setenv("XTQ_VIT_GROUP", "1")
+        st1, tr1 = hb.tailbite(X[:n], K, 147, 16, trellis=True)
+        assert torch.equal(st, st1) and torch.equal(tr, tr1), (K, n)
