@@ -1331,9 +1331,15 @@ __global__ __launch_bounds__(kFwdThreads) void tailbite_fused_kernel(
         const int q = t - nseq;
         if (tid == 0) {
             int ov = -1;
+            // relaxed polls, one acquire fence once the flag is seen: an
+            // acquire per poll invalidates the L2 that the other workgroups'
+            // passes of the XCD read their codebook and rows from (every
+            // waiting workgroup of a batch below one tile per CU polls for a
+            // whole pass)
             for (int it = 0;; ++it) {
-                if (__hip_atomic_load(&flags[q], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT) ==
+                if (__hip_atomic_load(&flags[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
                     epoch) {
+                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
                     ov = __hip_atomic_load(&ovbuf[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                     break;
                 }
