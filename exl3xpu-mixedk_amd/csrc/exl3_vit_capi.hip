@@ -694,12 +694,13 @@ int run_tailbite_noalloc(DevCtx& cx, const float* dX, int nseq, int K, Code code
 }
 
 // Relative cost of one tile of the chain kernel per K, for splitting the CUs
-// between groups: kernel times of the 5120x5120 sweep (344 / 319 / 309 /
-// 290 / 289 / 309 ms for K = 2..7), K = 7 raised by 2 % to the K=7 : K=5
-// ratio measured with both running side by side (c4's q at K=5, k and v at
-// K=7).
+// between groups: the 2560x4096 column chain's rates (356k / 381k / 407k /
+// 398k / 381k / 367k tiles/s for K = 2..7), K = 7 raised by 4 % to the
+// K=7 : K=5 ratio measured with both running side by side (5120 inputs, 6144
+// outputs at K=5 and 2048 at K=7: 0.721 against 0.640 ms a tile, where the
+// ratios of an earlier forward left K=7's launch 16 ms behind K=5's 418).
 double chain_tile_cost(int K) {
-    static const double c[8] = {1.0, 1.0, 1.11, 1.03, 1.0, 0.94, 0.94, 1.02};
+    static const double c[8] = {1.0, 1.0, 1.143, 1.068, 1.0, 1.023, 1.068, 1.153};
     return (K >= 2 && K <= 7) ? c[K] : 1.0;
 }
 
