@@ -988,34 +988,10 @@ int unpack_entry(const int16_t* d_trellis, int nt, int K, S* d_states, void* str
     return 0;
 }
 
-// The Hadamard entries (scales NULL: none).
-int had_left_entry(const float* d_ht, const float* d_in, float* d_out, int rows, int cols,
-                   const float* div_rows, const float* div_cols, const float* mul_rows,
-                   void* stream) {
-    if (!d_ht || !d_in || !d_out) return 12;
-    if (d_in == d_out) return 12;
-    if (rows <= 0 || cols <= 0 || rows % 128 || rows / 128 > 65535) return 6;
-    hipError_t e = xtq::launch_had_left(d_ht, d_in, d_out, rows, cols, div_rows, div_cols,
-                                        mul_rows, (hipStream_t)stream);
-    if (e != hipSuccess) {
-        fprintf(stderr, "xtq_vit had128: %s\n", hipGetErrorString(e));
-        return 4;
-    }
-    return 0;
-}
-
-int had_right_entry(const float* d_h, const float* d_in, float* d_out, int rows, int cols,
-                    const float* mul_cols, void* stream) {
-    if (!d_h || !d_in || !d_out) return 12;
-    if (d_in == d_out) return 12;
-    if (rows <= 0 || cols <= 0 || cols % 128 || (rows + 31) / 32 > 65535) return 6;
-    hipError_t e = xtq::launch_had_right(d_h, d_in, d_out, rows, cols, mul_cols,
-                                         (hipStream_t)stream);
-    if (e != hipSuccess) {
-        fprintf(stderr, "xtq_vit had128: %s\n", hipGetErrorString(e));
-        return 4;
-    }
-    return 0;
+int had_status(hipError_t e) {
+    if (e == hipSuccess) return 0;
+    fprintf(stderr, "xtq_vit had128: %s\n", hipGetErrorString(e));
+    return 4;
 }
 
 }  // namespace
@@ -1262,26 +1238,30 @@ int xtq_trellis_unpack64_dev(const int16_t* d_trellis, int nt, int K, int64_t* d
 
 int xtq_had128_left_dev(const float* d_ht, const float* d_in, float* d_out, int rows, int cols,
                         void* stream) {
-    return had_left_entry(d_ht, d_in, d_out, rows, cols, nullptr, nullptr, nullptr, stream);
-}
-
-int xtq_had128_left_scaled_dev(const float* d_ht, const float* d_in, float* d_out, int rows,
-                               int cols, const float* d_div_rows, const float* d_div_cols,
-                               const float* d_mul_rows, void* stream) {
-    if ((d_div_rows != nullptr) != (d_div_cols != nullptr) || (d_div_rows && d_mul_rows))
-        return 12;
-    return had_left_entry(d_ht, d_in, d_out, rows, cols, d_div_rows, d_div_cols, d_mul_rows,
-                          stream);
+    if (!d_ht || !d_in || !d_out) return 12;
+    if (d_in == d_out) return 12;
+    if (rows <= 0 || cols <= 0 || rows % 128 || rows / 128 > 65535) return 6;
+    return had_status(
+        xtq::launch_had_left(d_ht, d_in, d_out, rows, cols, (hipStream_t)stream));
 }
 
 int xtq_had128_right_dev(const float* d_h, const float* d_in, float* d_out, int rows, int cols,
                          void* stream) {
-    return had_right_entry(d_h, d_in, d_out, rows, cols, nullptr, stream);
+    if (!d_h || !d_in || !d_out) return 12;
+    if (d_in == d_out) return 12;
+    if (rows <= 0 || cols <= 0 || cols % 128 || (rows + 31) / 32 > 65535) return 6;
+    return had_status(
+        xtq::launch_had_right(d_h, d_in, d_out, rows, cols, (hipStream_t)stream));
 }
 
-int xtq_had128_right_scaled_dev(const float* d_h, const float* d_in, float* d_out, int rows,
-                                int cols, const float* d_mul_cols, void* stream) {
-    return had_right_entry(d_h, d_in, d_out, rows, cols, d_mul_cols, stream);
+int xtq_had128_both_dev(const float* d_h, const float* d_in, float* d_out, int rows, int cols,
+                        const float* d_row_scale, const float* d_col_scale, int divide,
+                        void* stream) {
+    if (!d_h || !d_in || !d_out || !d_row_scale || !d_col_scale) return 12;
+    if (d_in == d_out) return 12;
+    if (rows <= 0 || cols <= 0 || rows % 128 || cols % 128 || (rows + 31) / 32 > 65535) return 6;
+    return had_status(xtq::launch_had_both(d_h, d_in, d_out, rows, cols, d_row_scale, d_col_scale,
+                                           divide != 0, (hipStream_t)stream));
 }
 
 int xtq_vit_get_lut(const char* code, float* out) {

@@ -102,21 +102,23 @@ hipError_t launch_lfac_quads(const float* L, int k, float* Lq, hipStream_t strea
 // out = blockdiag(ht^T) @ in for in, out [rows][cols] fp32 row-major (rows a
 // multiple of 128, in != out), ht[t][r] the weight of input row t in output
 // row r: each output one fp32 fused multiply-add chain in ascending order.
-// With div_rows [rows] and div_cols [cols] the input is first divided by its
-// row's and then by its column's scale; with mul_rows [rows] the output is
-// multiplied by its row's (NULL: not).
 hipError_t launch_had_left(const float* ht, const float* in, float* out, int rows, int cols,
-                           const float* div_rows, const float* div_cols, const float* mul_rows,
                            hipStream_t stream);
 
 // out = in @ blockdiag(h) for in, out [rows][cols] fp32 row-major (cols a
 // multiple of 128, in != out), h[t][c] the weight of input column t in
 // output column c: each output one fp32 fused multiply-add chain in
 // ascending order (the products and order of launch_had_left on the
-// transpose).  With mul_cols [cols] the output is multiplied by its column's
-// scale (NULL: not).
+// transpose).
 hipError_t launch_had_right(const float* h, const float* in, float* out, int rows, int cols,
-                            const float* mul_cols, hipStream_t stream);
+                            hipStream_t stream);
+
+// Both, in that order, of in / row_scale / col_scale (divide), or with the
+// left transform multiplied by row_scale and the right one by col_scale; rows
+// and cols multiples of 128.
+hipError_t launch_had_both(const float* h, const float* in, float* out, int rows, int cols,
+                           const float* row_scale, const float* col_scale, bool divide,
+                           hipStream_t stream);
 
 // The BlockLDLQ sweep of the column tiles jc0 .. jc0+tnl-1 of W [k][n]
 // (inner domain, row-major, k and n multiples of 16) as one persistent

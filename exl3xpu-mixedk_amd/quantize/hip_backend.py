@@ -67,8 +67,7 @@ def lib():
         L.xtq_vit_get_lut.argtypes = [cp, vp]
         L.xtq_had128_left_dev.argtypes = [vp, vp, vp, i32, i32, vp]
         L.xtq_had128_right_dev.argtypes = [vp, vp, vp, i32, i32, vp]
-        L.xtq_had128_left_scaled_dev.argtypes = [vp, vp, vp, i32, i32, vp, vp, vp, vp]
-        L.xtq_had128_right_scaled_dev.argtypes = [vp, vp, vp, i32, i32, vp, vp]
+        L.xtq_had128_both_dev.argtypes = [vp, vp, vp, i32, i32, vp, vp, i32, vp]
         L.xtq_vit_scratch_per_seq.argtypes = [i32]
         L.xtq_vit_scratch_per_seq.restype = i64
         L.xtq_vit_chunk_seqs.argtypes = [i32, i32, ctypes.POINTER(ctypes.c_int)]
@@ -87,8 +86,7 @@ def lib():
                    "xtq_trellis_decode_dev", "xtq_trellis_pack_dev",
                    "xtq_trellis_unpack_dev", "xtq_trellis_pack64_dev",
                    "xtq_trellis_unpack64_dev", "xtq_vit_get_lut", "xtq_had128_left_dev",
-                   "xtq_had128_right_dev", "xtq_had128_left_scaled_dev",
-                   "xtq_had128_right_scaled_dev"):
+                   "xtq_had128_right_dev", "xtq_had128_both_dev"):
             getattr(L, fn).restype = i32
         _LIB = L
     return _LIB
@@ -261,69 +259,76 @@ def decode(trellis: torch.Tensor, K: int, code: str = "mul1",
     return out
 
 
-def _scale(v: torch.Tensor | None, n: int, w: torch.Tensor, name: str):
-    """A channel scale as the contiguous fp32 [n] vector the kernels read."""
-    if v is None:
-        return None
-    if v.shape != (n,) or v.device != w.device:
-        raise ValueError(f"{name} must be [{n}] on {w.device}, got {tuple(v.shape)} on {v.device}")
-    return _dev_tensor(v, torch.float32, name)
-
-
-def had128_left(w: torch.Tensor, h: torch.Tensor, div_rows: torch.Tensor | None = None,
-                div_cols: torch.Tensor | None = None,
-                mul_rows: torch.Tensor | None = None) -> torch.Tensor:
+def had128_left(w: torch.Tensor, h: torch.Tensor) -> torch.Tensor:
     """blockdiag(h) @ w for w [k, n] fp32 (device, k a multiple of 128) and
     any 128x128 h on the same device (the reference applies the normalised
     Sylvester matrix): each output one fused multiply-add chain in ascending
     order, as torch's CPU sgemm evaluates the reference's matmul
-    (xtq_had128_left_dev, which takes the multipliers by input row, h^T).
-    div_rows [k] with div_cols [n]: of w / div_rows[:, None] / div_cols;
-    mul_rows [k]: times mul_rows[:, None], rounded as separate passes are
-    (xtq_had128_left_scaled_dev)."""
+    (xtq_had128_left_dev, which takes the multipliers by input row, h^T)."""
     w = _dev_tensor(w, torch.float32, "w")
     h = _dev_tensor(h, torch.float32, "h")
     if w.dim() != 2 or w.shape[0] % 128 or h.shape != (128, 128) or h.device != w.device:
         raise ValueError(f"had128_left needs w [128m, n] and h [128, 128] on one device, got "
                          f"{tuple(w.shape)}, {tuple(h.shape)}")
-    dr = _scale(div_rows, w.shape[0], w, "div_rows")
-    dc = _scale(div_cols, w.shape[1], w, "div_cols")
-    mr = _scale(mul_rows, w.shape[0], w, "mul_rows")
     out = torch.empty_like(w)
     if w.numel() == 0:
         return out
     with torch.cuda.device(w.device):
         ht = h.t().contiguous()
-        rc = lib().xtq_had128_left_scaled_dev(
-            ht.data_ptr(), w.data_ptr(), out.data_ptr(), w.shape[0], w.shape[1],
-            dr.data_ptr() if dr is not None else None, dc.data_ptr() if dc is not None else None,
-            mr.data_ptr() if mr is not None else None, _stream(w.device))
-    _check("xtq_had128_left_scaled_dev", rc)
+        rc = lib().xtq_had128_left_dev(ht.data_ptr(), w.data_ptr(), out.data_ptr(), w.shape[0],
+                                       w.shape[1], _stream(w.device))
+    _check("xtq_had128_left_dev", rc)
     return out
 
 
-def had128_right(w: torch.Tensor, h: torch.Tensor,
-                 mul_cols: torch.Tensor | None = None) -> torch.Tensor:
+def had128_right(w: torch.Tensor, h: torch.Tensor) -> torch.Tensor:
     """w @ blockdiag(h) for w [k, n] fp32 (device, n a multiple of 128) and
     any 128x128 h on the same device: each output one fused multiply-add
     chain in ascending order, as torch's CPU sgemm evaluates the reference's
-    matmul (xtq_had128_right_dev).  mul_cols [n]: times mul_cols, rounded as
-    a separate pass is (xtq_had128_right_scaled_dev)."""
+    matmul (xtq_had128_right_dev)."""
     w = _dev_tensor(w, torch.float32, "w")
     h = _dev_tensor(h, torch.float32, "h")
     if w.dim() != 2 or w.shape[1] % 128 or h.shape != (128, 128) or h.device != w.device:
         raise ValueError(f"had128_right needs w [k, 128m] and h [128, 128] on one device, got "
                          f"{tuple(w.shape)}, {tuple(h.shape)}")
-    mc = _scale(mul_cols, w.shape[1], w, "mul_cols")
     out = torch.empty_like(w)
     if w.numel() == 0:
         return out
     with torch.cuda.device(w.device):
         hc = h.contiguous()
-        rc = lib().xtq_had128_right_scaled_dev(
-            hc.data_ptr(), w.data_ptr(), out.data_ptr(), w.shape[0], w.shape[1],
-            mc.data_ptr() if mc is not None else None, _stream(w.device))
-    _check("xtq_had128_right_scaled_dev", rc)
+        rc = lib().xtq_had128_right_dev(hc.data_ptr(), w.data_ptr(), out.data_ptr(), w.shape[0],
+                                        w.shape[1], _stream(w.device))
+    _check("xtq_had128_right_dev", rc)
+    return out
+
+
+def had128_both(w: torch.Tensor, h: torch.Tensor, rows: torch.Tensor, cols: torch.Tensor,
+                divide: bool) -> torch.Tensor:
+    """Both transforms of w [k, n] fp32 (device, k and n multiples of 128)
+    and its scales rows [k], cols [n] in one pass, rounded as had128_left,
+    had128_right and a pass per scale are (xtq_had128_both_dev): divide gives
+    had_right(had_left(w / rows[:, None] / cols)), else
+    had_right(had_left(w) * rows[:, None]) * cols."""
+    w = _dev_tensor(w, torch.float32, "w")
+    h = _dev_tensor(h, torch.float32, "h")
+    if (w.dim() != 2 or w.shape[0] % 128 or w.shape[1] % 128 or h.shape != (128, 128)
+            or h.device != w.device):
+        raise ValueError(f"had128_both needs w [128a, 128b] and h [128, 128] on one device, got "
+                         f"{tuple(w.shape)}, {tuple(h.shape)}")
+    for v, n, name in ((rows, w.shape[0], "rows"), (cols, w.shape[1], "cols")):
+        if v.shape != (n,) or v.device != w.device:
+            raise ValueError(f"{name} must be [{n}] on {w.device}, got {tuple(v.shape)} on "
+                             f"{v.device}")
+    rows = _dev_tensor(rows, torch.float32, "rows")
+    cols = _dev_tensor(cols, torch.float32, "cols")
+    out = torch.empty_like(w)
+    if w.numel() == 0:
+        return out
+    with torch.cuda.device(w.device):
+        rc = lib().xtq_had128_both_dev(h.data_ptr(), w.data_ptr(), out.data_ptr(), w.shape[0],
+                                       w.shape[1], rows.data_ptr(), cols.data_ptr(), int(divide),
+                                       _stream(w.device))
+    _check("xtq_had128_both_dev", rc)
     return out
 
 

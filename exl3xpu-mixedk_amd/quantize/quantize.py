@@ -183,9 +183,8 @@ def to_inner(w_orig: torch.Tensor, suh: torch.Tensor, svh: torch.Tensor,
              h: torch.Tensor) -> torch.Tensor:
     """W_orig [k, n] -> W_inner = B_k diag(1/suh) W diag(1/svh) B_n."""
     if _fold_scales(w_orig, suh, svh):
-        hd = h.to(w_orig.device, torch.float32)
-        w = _hb.had128_left(w_orig.contiguous(), hd, div_rows=suh.float(), div_cols=svh.float())
-        return _hb.had128_right(w, hd)
+        return _hb.had128_both(w_orig.contiguous(), h.to(w_orig.device, torch.float32),
+                               suh.float(), svh.float(), divide=True)
     w = w_orig / suh.float().unsqueeze(1)
     w = w / svh.float().unsqueeze(0)
     return had_right(had_left(w, h), h)
@@ -195,9 +194,8 @@ def from_inner(w_inner: torch.Tensor, suh: torch.Tensor, svh: torch.Tensor,
                h: torch.Tensor) -> torch.Tensor:
     """W_inner -> W_orig = diag(suh) B_k W_i B_n diag(svh)."""
     if _fold_scales(w_inner, suh, svh):
-        hd = h.to(w_inner.device, torch.float32)
-        w = _hb.had128_left(w_inner.contiguous(), hd, mul_rows=suh.float())
-        return _hb.had128_right(w, hd, mul_cols=svh.float())
+        return _hb.had128_both(w_inner.contiguous(), h.to(w_inner.device, torch.float32),
+                               suh.float(), svh.float(), divide=False)
     w = had_left(w_inner, h) * suh.float().unsqueeze(1)
     return had_right(w, h) * svh.float().unsqueeze(0)
 

@@ -276,18 +276,6 @@ XTQ_API int xtq_trellis_unpack64_dev(const int16_t* d_trellis, int nt, int K, in
  */
 XTQ_API int xtq_had128_left_dev(const float* d_ht, const float* d_in, float* d_out, int rows,
                                 int cols, void* stream);
-/*
- * xtq_had128_left_dev with the channel scales of to_inner / from_inner
- * (quantize.py:148-163) in the same pass, each rounded as a pass of its own:
- * d_div_rows [rows] with d_div_cols [cols] (both or neither): the input is
- * divided by its row's scale, then by its column's, before the transform;
- * d_mul_rows [rows] (not with the divisors): the output is multiplied by its
- * row's scale.
- */
-XTQ_API int xtq_had128_left_scaled_dev(const float* d_ht, const float* d_in, float* d_out,
-                                       int rows, int cols, const float* d_div_rows,
-                                       const float* d_div_cols, const float* d_mul_rows,
-                                       void* stream);
 
 /*
  * Device-pointer block-128 transform on the last dimension: the HIP
@@ -302,11 +290,19 @@ XTQ_API int xtq_had128_left_scaled_dev(const float* d_ht, const float* d_in, flo
  */
 XTQ_API int xtq_had128_right_dev(const float* d_h, const float* d_in, float* d_out, int rows,
                                  int cols, void* stream);
-/* xtq_had128_right_dev with the output multiplied by its column's scale
- * d_mul_cols [cols] (NULL: not). */
-XTQ_API int xtq_had128_right_scaled_dev(const float* d_h, const float* d_in, float* d_out,
-                                        int rows, int cols, const float* d_mul_cols,
-                                        void* stream);
+/*
+ * to_inner (divide != 0) and from_inner (divide == 0) of quantize.py:148-163
+ * in one pass: both of the transforms above with multipliers d_h, of
+ * [rows][cols] fp32 row-major buffers (both multiples of 128, rows up to
+ * 2,097,120, d_out not d_in).  divide: the input is divided by its row's
+ * scale d_row_scale [rows], then by its column's d_col_scale [cols], before
+ * the transforms; else the first-dimension transform's result is multiplied
+ * by its row's scale and the last one's by its column's.  Every quotient,
+ * product and sum rounds as in passes of its own.  Stream-ordered.
+ */
+XTQ_API int xtq_had128_both_dev(const float* d_h, const float* d_in, float* d_out, int rows,
+                                int cols, const float* d_row_scale, const float* d_col_scale,
+                                int divide, void* stream);
 
 /*
  * Copies the fp32 decode table of `code` (65536 entries) into host memory

@@ -32,6 +32,20 @@ def test_scaled_transforms_match_cpu(xq, k, n):
     assert torch.equal(xq.to_inner(w.cuda(), sud.double(), svd.double(), hd).cpu(), want_in)
 
 
+def test_scaled_transforms_more_blocks_than_workgroups(xq):
+    """17 x 17 blocks (a second round for 33 of the 256 workgroups) and
+    multipliers that are not symmetric."""
+    k = n = 17 * 128
+    g = torch.Generator().manual_seed(17)
+    w = torch.randn(k, n, generator=g)
+    su = torch.randn(k, generator=g) + 3.0
+    sv = torch.randn(n, generator=g) + 3.0
+    h = torch.randn(128, 128, generator=g) / 11.0
+    dev = [t.cuda() for t in (w, su, sv, h)]
+    assert torch.equal(xq.to_inner(*dev).cpu(), xq.to_inner(w, su, sv, h))
+    assert torch.equal(xq.from_inner(*dev).cpu(), xq.from_inner(w, su, sv, h))
+
+
 @pytest.mark.parametrize("cols", (1, 63, 64, 65, 200))
 def test_had_left_ragged_columns(xq, cols):
     """Column counts around the kernel's 64-column tiles, and more tiles than
