@@ -459,14 +459,15 @@ double fused_steps(int n, int d1, int d2, int ncu) {
 // the separate launches (with XTQ_VIT_GROUP set: below 4 sequences per CU, as
 // a group asks for separate launches above).  The fused launch runs one
 // sequence per workgroup, traces back inside (the time of about 7 and 16
-// steps; at K=2, whose rows are 4 KiB, 24 and 48) and fills its rounds with 2n
-// passes; separate launches run T sequences per
-// workgroup (1.17 against 1.33 us per step and sequence at K=4) and read all
-// backpointer rows again: one sequence's tracebacks take 0.03 (K=7) to 0.1 ms
-// (K=2), more of them 4.7 TB/s, up to the 0.3 ms of one-lane tracebacks.  Measured, fused / separate, ms: K=4 320 tiles
-// 1.07 / 1.36, 512 1.42 / 1.39, 768 2.09 / 2.21, 1003 2.78 / 2.53, 1100 3.10 /
-// 3.69, 2100 5.91 / 7.67; K=7 1003 3.00 / 2.67; K=2 64 0.81 / 0.87, 3700 11.8 /
-// 11.0.
+// steps; at K=2, whose rows are 4 KiB, 12 and 26, or 25 and 50 once half the
+// CUs read them at the same time) and fills its rounds with 2n passes; separate
+// launches run T sequences per workgroup (1.17 against 1.33 us per step and
+// sequence at K=4) and read all backpointer rows again: one sequence's
+// tracebacks take 0.025 (K=7) to 0.05 ms (K=2), more of them 4.7 TB/s, up to
+// the 0.3 ms of one-lane tracebacks.  Measured, fused / separate, ms: K=4 256
+// tiles 0.72 / 0.75, 300 1.04 / 1.32, 400 1.37 / 1.33, 768 2.07 / 2.17, 1003
+// 2.74 / 2.50, 2000 5.51 / 5.00; K=7 1003 2.99 / 2.66; K=2 1 0.73 / 0.76, 64
+// 0.775 / 0.774, 128 0.81 / 0.78, 512 1.60 / 1.57.
 bool use_fused(const DevCtx& cx, int K, int n, int n1) {
     if (const char* e = getenv("XTQ_VIT_FUSED")) {
         if (!strcmp(e, "0")) return false;
@@ -477,11 +478,12 @@ bool use_fused(const DevCtx& cx, int K, int n, int n1) {
     // (beyond, a round is a small part of the whole and T decides)
     if (n >= 16 * ncu) return false;
     double rows = 1.5e-6 / 4.7 * (double)xtq::bp_tile_bytes(K) * n;      // us
-    const double lat = 25.0 + 75.0 * (double)xtq::bp_step_bytes(K) / 4096.0;
+    const double lat = 22.0 + 28.0 * (double)xtq::bp_step_bytes(K) / 4096.0;
     rows = rows < lat ? lat : rows > 300.0 ? 300.0 : rows;
     const double split =
         xtq::forward_cost_us(K, xtq::forward_group(K, n, ncu), n, ncu) * (n1 + xtq::kSteps);
-    const int tb1 = K == 2 ? 24 : 7, tb2 = K == 2 ? 48 : 16;     // steps' time per traceback
+    // steps' time per traceback
+    const int tb1 = K > 2 ? 7 : 2 * n < ncu ? 12 : 25, tb2 = K > 2 ? 16 : 2 * n < ncu ? 26 : 50;
     return fused_steps(n, n1 + tb1, xtq::kSteps + tb2, ncu) * xtq::forward_step_us(K, 1) <=
            split + rows + 50.0;
 }

@@ -13,7 +13,7 @@ namespace xtq {
 // 256-step sequences in lockstep, 64 trellis states per thread per sequence.
 constexpr int kFwdThreads = 1024;
 // Threads per traceback workgroup.
-constexpr int kTbThreads = 256;
+constexpr int kTbThreads = 512;
 // Number of trellis steps per sequence (16x16 tile).
 constexpr int kSteps = 256;
 // Backpointer slots stored per sequence: steps 1..255 of a pass.

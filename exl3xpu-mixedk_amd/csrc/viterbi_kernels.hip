@@ -790,80 +790,57 @@ __device__ __forceinline__ int chase_links(const uint8_t* stage, int hi, int lo,
               : chase_links<K, false>(stage, hi, lo, st, s);
 }
 
-// Traceback of one sequence by the calling workgroup: from cur = s_{nsteps-1}
-// (shared; set by the caller before a barrier) down to step `stop`.  The
-// backpointer slots stop .. nsteps-2 (slot i-1 links s_i to s_{i-1}) are
-// staged through `stage` in coalesced 16-byte loads by all threads, and one
-// thread chases the links in LDS.  On return (after a barrier) cur = s_stop
-// and st[i] = s_i for stop <= i <= nsteps-2 when st is non-null.
-template <int K>
-__device__ __forceinline__ void tb_chase(const uint8_t* __restrict__ bpq, int nsteps, int stop,
-                                         uint4* stage, int stage_bytes, int32_t* st,
-                                         int32_t& cur) {
-    using G = Geom<K>;
-    const int tid = threadIdx.x, nthr = blockDim.x;
-    const int ch = stage_bytes / G::BPSTEP;  // slots per staged chunk
-    for (int hi = nsteps - 2; hi >= stop; ) {
-        const int lo = (hi - ch + 1 > stop) ? hi - ch + 1 : stop;
-        const int n16 = (hi - lo + 1) * (G::BPSTEP / 16);
-        const uint4* src = (const uint4*)(bpq + (size_t)lo * G::BPSTEP);
-        __syncthreads();
-        for (int k = tid; k < n16; k += nthr) stage[k] = src[k];
-        __syncthreads();
-        if (tid == 0) cur = chase_links<K>((const uint8_t*)stage, hi, lo, st, cur);
-        hi = lo - 1;
-    }
-    __syncthreads();
-}
+// Traceback of one sequence by the calling workgroup of NT threads: from
+// cur = s_{nsteps-1} (shared; set by the caller before a barrier) down to step
+// `stop`.  The backpointer slots stop .. nsteps-2 (slot i-1 links s_i to
+// s_{i-1}) are staged through `stage` (64 NT bytes) in coalesced 16-byte loads
+// by all threads, the next two chunks' loads in flight in registers while
+// thread 0 chases the current chunk's links in LDS (per chunk: store, barrier,
+// issue the load two chunks ahead, chase), so the chase rather than the load
+// latency sets the pace.  On return (after a barrier) cur = s_stop and st[i] = s_i for
+// stop <= i <= nsteps-2 when st is non-null.
+constexpr int kTbStage = 64 * kFwdThreads;
 
-// tb_chase for a 1024-thread workgroup with a fixed 64 KiB staging area and
-// the next two chunks' loads in flight in registers while thread 0 chases
-// the current chunk (per chunk: store, barrier, issue the load two chunks
-// ahead, chase), so the chase rather than the load latency sets the pace.
-// Same contract as tb_chase.
-constexpr int kTbStage = 65536;
-
-// Loads chunk c (slots lo .. hi, 64 KiB at most) of a tb_chase_pf run into
+// Loads chunk c (slots lo .. hi, 64 NT bytes at most) of a tb_chase_pf run into
 // this thread's four registers.
-template <int K>
+template <int K, int NT>
 __device__ __forceinline__ void tb_chunk_load(const uint8_t* __restrict__ bpq, int nsteps,
                                               int stop, int nc, int c, int tid, uint4& r0,
                                               uint4& r1, uint4& r2, uint4& r3) {
     using G = Geom<K>;
-    constexpr int CH = kTbStage / G::BPSTEP;
+    constexpr int CH = 64 * NT / G::BPSTEP;
     if (c >= nc) return;
     const int hi = nsteps - 2 - c * CH, lo = (hi - CH + 1 > stop) ? hi - CH + 1 : stop;
     const int n16 = (hi - lo + 1) * (G::BPSTEP / 16);
     const uint4* src = (const uint4*)(bpq + (size_t)lo * G::BPSTEP);
     if (tid < n16) r0 = src[tid];
-    if (tid + kFwdThreads < n16) r1 = src[tid + kFwdThreads];
-    if (tid + 2 * kFwdThreads < n16) r2 = src[tid + 2 * kFwdThreads];
-    if (tid + 3 * kFwdThreads < n16) r3 = src[tid + 3 * kFwdThreads];
+    if (tid + NT < n16) r1 = src[tid + NT];
+    if (tid + 2 * NT < n16) r2 = src[tid + 2 * NT];
+    if (tid + 3 * NT < n16) r3 = src[tid + 3 * NT];
 }
 
-template <int K>
+template <int K, int NT = kFwdThreads>
 __device__ __forceinline__ void tb_chase_pf(const uint8_t* __restrict__ bpq, int nsteps,
                                             int stop, uint4* stage, int32_t* st,
                                             int32_t& cur) {
     using G = Geom<K>;
-    constexpr int CH = kTbStage / G::BPSTEP;           // slots per chunk
-    static_assert(kTbStage / 16 == 4 * kFwdThreads, "four uint4 per thread per chunk");
+    constexpr int CH = 64 * NT / G::BPSTEP;           // slots per chunk
     const int tid = threadIdx.x;
     const int nc = (nsteps - 1 - stop + CH - 1) / CH;  // slots stop .. nsteps-2
     uint4 a0, a1, a2, a3, b0, b1, b2, b3;
-    tb_chunk_load<K>(bpq, nsteps, stop, nc, 0, tid, a0, a1, a2, a3);
-    tb_chunk_load<K>(bpq, nsteps, stop, nc, 1, tid, b0, b1, b2, b3);
+    tb_chunk_load<K, NT>(bpq, nsteps, stop, nc, 0, tid, a0, a1, a2, a3);
+    tb_chunk_load<K, NT>(bpq, nsteps, stop, nc, 1, tid, b0, b1, b2, b3);
     for (int c = 0; c < nc; ++c) {
         const int hi = nsteps - 2 - c * CH, lo = (hi - CH + 1 > stop) ? hi - CH + 1 : stop;
         const int n16 = (hi - lo + 1) * (G::BPSTEP / 16);
         __syncthreads();                                // previous chase done with stage
         if (tid < n16) stage[tid] = a0;
-        if (tid + kFwdThreads < n16) stage[tid + kFwdThreads] = a1;
-        if (tid + 2 * kFwdThreads < n16) stage[tid + 2 * kFwdThreads] = a2;
-        if (tid + 3 * kFwdThreads < n16) stage[tid + 3 * kFwdThreads] = a3;
+        if (tid + NT < n16) stage[tid + NT] = a1;
+        if (tid + 2 * NT < n16) stage[tid + 2 * NT] = a2;
+        if (tid + 3 * NT < n16) stage[tid + 3 * NT] = a3;
         __syncthreads();
         a0 = b0; a1 = b1; a2 = b2; a3 = b3;
-        tb_chunk_load<K>(bpq, nsteps, stop, nc, c + 2, tid, b0, b1, b2, b3);
+        tb_chunk_load<K, NT>(bpq, nsteps, stop, nc, c + 2, tid, b0, b1, b2, b3);
         if (tid == 0) cur = chase_links<K>((const uint8_t*)stage, hi, lo, st, cur);
     }
     __syncthreads();
@@ -888,32 +865,38 @@ __device__ __forceinline__ void store_word(int16_t* o, uint32_t word) {
     o[1] = (int16_t)(uint16_t)(word >> 16);
 }
 
+// Traceback of a run with its own launch, one workgroup per sequence: bound by
+// the chase up to one sequence per CU, by the rows' bytes (4.7 TB/s) from two.
+// 512 threads and 32 KiB of staging: four workgroups per CU, as before, whose
+// loads are now two chunks ahead of the chase (256 threads that waited for each
+// chunk's loads before: 1 / 256 / 512 / 1500 / 2001 sequences of 256 steps, us,
+// K=4 31 / 52 / 60 / 202 / 221 -> 23 / 26 / 42 / 160 / 203, K=2 85 / 97 / 161 /
+// 390 / 430 -> 33 / 42 / 98 / 312 / 405; with 1024 threads and two workgroups
+// per CU K=2's 1 and 64 take 28, K=7's 1003 and more take 40 % longer).
 template <int K>
-__global__ __launch_bounds__(kTbThreads) void tb_kernel(
+__global__ __launch_bounds__(kTbThreads, 8) void tb_kernel(
     const uint8_t* __restrict__ bp, const int32_t* __restrict__ send, int nsteps, int stop,
     int shift, int32_t* __restrict__ sout, int32_t* __restrict__ states,
     int16_t* __restrict__ trellis) {
     using G = Geom<K>;
-    constexpr int STAGE = 32768;
-    __shared__ uint4 stage[STAGE / 16];
+    static_assert(kTbThreads >= kSteps + 8 * 7, "a thread per state and packed word");
+    __shared__ uint4 stage[4 * kTbThreads];
     __shared__ int32_t st[kSteps];
     __shared__ int32_t cur;
 
     const int q = blockIdx.x, tid = threadIdx.x;
-    const uint8_t* bpq = bp + (size_t)q * ((size_t)kSlots * G::BPSTEP);
     const bool keep = (states != nullptr) || (trellis != nullptr);
     if (tid == 0) {
         cur = send[q] & 0xFFFF;
         if (keep) st[nsteps - 1] = cur;
     }
-    tb_chase<K>(bpq, nsteps, stop, stage, STAGE, keep ? st : nullptr, cur);
+    tb_chase_pf<K, kTbThreads>(bp + (size_t)q * ((size_t)kSlots * G::BPSTEP), nsteps, stop, stage,
+                   keep ? st : nullptr, cur);
     if (sout && tid == 0) sout[q] = cur >> shift;
-    if (states) {
-        for (int t = tid; t < nsteps; t += kTbThreads) states[(size_t)q * nsteps + t] = st[t];
-    }
-    if (trellis && nsteps == kSteps) {
-        for (int wd = tid; wd < 8 * K; wd += kTbThreads)
-            store_word(trellis + (size_t)q * 16 * K + 2 * wd, pack_word<K>(st, wd));
+    if (states && tid < nsteps) states[(size_t)q * nsteps + tid] = st[tid];
+    if (trellis && nsteps == kSteps && tid >= kSteps && tid < kSteps + 8 * K) {
+        const int wd = tid - kSteps;
+        store_word(trellis + (size_t)q * 16 * K + 2 * wd, pack_word<K>(st, wd));
     }
 }
 
@@ -1288,8 +1271,8 @@ __global__ __launch_bounds__(kTbLaneSeqs) void tb_defer_kernel(
 // pass-1 slots (pass 1 has finished reading them before it publishes) and are
 // traced back in the same workgroup, which writes the states and the packed
 // trellis: the 1024-thread chase with its loads two chunks ahead
-// (tb_chase_pf) takes 20-30 us where a tb_kernel launch after the passes took
-// 86 (64 tiles, K=2) to 108 us (1003 tiles, K=5) and its gap.
+// (tb_chase_pf) takes 20-30 us and saves the launches and gaps of separate
+// tracebacks (64 tiles at K=4 0.68 ms, with separate launches 0.75).
 template <int K>
 __global__ __launch_bounds__(kFwdThreads) void tailbite_fused_kernel(
     const float* __restrict__ X, int nseq, const float* __restrict__ lut, int pivot,

@@ -552,3 +552,21 @@ def test_batch_route_edges(hb, K, monkeypatch):
         monkeypatch.setenv("XTQ_VIT_GROUP", "1")
         st1, tr1 = hb.tailbite(X[:n], K, 147, 16, trellis=True)
         assert torch.equal(st, st1) and torch.equal(tr, tr1), (K, n)
+
+
+@pytest.mark.parametrize("K", range(2, 8))
+def test_traceback_chunk_edges(hb, oracle_mod, mul1_lut, K):
+    """One-workgroup tracebacks around the ends of their 32 KiB chunks (8 rows
+    at K=2, 64 at K=7): whole runs, and runs traced back to a step next to the
+    last one, to a chunk's edge and to the start."""
+    rows = (32 << 10) // (4096, 4096, 2048, 2048, 1024, 512)[K - 2]
+    rng = np.random.default_rng(K)
+    for T in sorted({1, 2, rows, rows + 1, rows + 2, min(256, 2 * rows + 1), 256}):
+        X = rng.standard_normal((3, T)).astype(np.float32)
+        Xd = torch.from_numpy(X).cuda()
+        np.testing.assert_array_equal(hb.viterbi(Xd, K).cpu().numpy(),
+                                      oracle_mod.viterbi(X, mul1_lut, K, 16), err_msg=f"T={T}")
+        for bf in sorted({0, T - 1, max(0, T - 2), max(0, T - 1 - rows), max(0, T - 2 - rows)}):
+            np.testing.assert_array_equal(
+                hb.viterbi(Xd, K, back_from=bf).cpu().numpy(),
+                oracle_mod.viterbi(X, mul1_lut, K, 16, back_from=bf), err_msg=f"T={T} {bf}")
