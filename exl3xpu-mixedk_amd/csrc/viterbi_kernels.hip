@@ -304,7 +304,8 @@ constexpr bool kRematLane = (T == 1 && K <= 3);
 // computed after the barrier instead: 371k/395k/394k).  K = 2 gains nothing
 // and K = 6, 7, whose units belong to one group, lose 2-3 % (382k -> 371k,
 // 368k -> 363k).  With more sequences per workgroup the other sequences'
-// work already fills those slots.
+// work already fills those slots.  The plain and the fused forward have the
+// registers for them only with their one sequence a constant (see fwd_kernel).
 template <int K, int T>
 constexpr int kPreUnits = (T == 1 && K >= 3 && K <= 5) ? 2 : 0;
 template <int K, int T>
@@ -725,8 +726,15 @@ __global__ __launch_bounds__(kFwdThreads) void fwd_kernel(
     const bool pinned = (ov_in != nullptr);
     if (threadIdx.x < T)
         sm.ovs[threadIdx.x] = (pinned && (int)threadIdx.x < ntile) ? ov_in[q0 + threadIdx.x] : -1;
-    fwd_run<K, T>(sm, X, xstride, xlen, q0, ntile, lut, roll, nsteps, store_lo, pinned, bp,
-                  send + q0, err, (int)threadIdx.x);
+    // T = 1: a grid of nseq workgroups, so ntile is 1; as a constant it takes
+    // the loop over the sequences out, beside which the squares of kPreUnits
+    // do not fit the registers (2 to 5 spilled and reloaded in every step).
+    // A viterbi() call of 64 sequences at K = 2..7, with ntile a variable /
+    // the constant, us: 429 / 411, 468 / 395, 424 / 369, 441 / 375, 413 / 386,
+    // 426 / 396 (485, 493, 438, 433, 426, 441 without kPreUnits, the target in
+    // an SGPR).
+    fwd_run<K, T>(sm, X, xstride, xlen, q0, T == 1 ? 1 : ntile, lut, roll, nsteps, store_lo,
+                  pinned, bp, send + q0, err, (int)threadIdx.x);
 }
 
 // ---------------------------------------------------------------- traceback
