@@ -18,6 +18,7 @@
 #include <vector>
 
 #include "../../include/exl3_vit.h"
+#include "route.h"
 #include "viterbi_kernels.h"
 
 namespace {
@@ -414,12 +415,12 @@ int finish(DevCtx& cx, hipStream_t s) {
 }
 
 int pick_group(const DevCtx& cx, int K, int n) {
-    int T = xtq::forward_group(K, n, cx.ncu);
+    const int cap = xtq::forward_group_max(K);
+    int T = xtq::forward_group(K, cap, n, cx.ncu);
     if (const char* g = getenv("XTQ_VIT_GROUP")) {
         // Test hook: force the sequences per workgroup (1, 2, 4 or 8), clamped
         // to what the LDS footprint for K allows.
         const int want = atoi(g);
-        const int cap = xtq::forward_group_max(K);
         if (want == 1 || want == 2 || want == 4 || want == 8) T = want < cap ? want : cap;
     }
     return T;
@@ -437,55 +438,18 @@ int scratch_end(DevCtx& cx, hipStream_t s, bool sync) {
     return sync ? finish(cx, s) : 0;
 }
 
-// Steps until the last of a fused launch's 2n workgroups ends: each CU takes
-// the next of n first passes and then of n second passes, of d1 and d2 steps,
-// as soon as it is free.
-double fused_steps(int n, int d1, int d2, int ncu) {
-    const int r = n / ncu, m = n % ncu;        // pass 1: m CUs take r + 1, the others r
-    const int cus[2] = {ncu - m, m};
-    double t[2] = {(double)r * d1, (double)(r + 1) * d1};
-    double end = m ? t[1] : t[0];
-    for (int left = n; left > 0;) {
-        const int g = m && t[1] < t[0] ? 1 : 0;            // the CUs free first
-        t[g] = (t[g] < d1 ? d1 : t[g]) + d2;               // (a pass 2 waits for its pass 1)
-        if (t[g] > end) end = t[g];
-        left -= cus[g];
-    }
-    return end;
-}
-
 // Whether a chunk of n sequences runs as one fused two-pass launch:
 // XTQ_VIT_FUSED=0 never, =1 always, unset: if it is estimated to end before
 // the separate launches (with XTQ_VIT_GROUP set: below 4 sequences per CU, as
-// a group asks for separate launches above).  The fused launch runs one
-// sequence per workgroup, traces back inside (the time of about 7 and 16
-// steps; at K=2, whose rows are 4 KiB, 12 and 26, or 25 and 50 once half the
-// CUs read them at the same time) and fills its rounds with 2n passes; separate
-// launches run T sequences per workgroup (1.17 against 1.33 us per step and
-// sequence at K=4) and read all backpointer rows again: one sequence's
-// tracebacks take 0.025 (K=7) to 0.05 ms (K=2), more of them 4.7 TB/s, up to
-// the 0.3 ms of one-lane tracebacks.  Measured, fused / separate, ms: K=4 256
-// tiles 0.72 / 0.75, 300 1.04 / 1.32, 400 1.37 / 1.33, 768 2.07 / 2.17, 1003
-// 2.74 / 2.50, 2000 5.51 / 5.00; K=7 1003 2.99 / 2.66; K=2 1 0.73 / 0.76, 64
-// 0.775 / 0.774, 128 0.81 / 0.78, 512 1.60 / 1.57.
-bool use_fused(const DevCtx& cx, int K, int n, int n1) {
+// a group asks for separate launches above).
+bool use_fused(const DevCtx& cx, int K, int n, int n1, int pivot) {
     if (const char* e = getenv("XTQ_VIT_FUSED")) {
         if (!strcmp(e, "0")) return false;
         if (!strcmp(e, "1")) return true;
     }
-    const int ncu = cx.ncu > 0 ? cx.ncu : 1;
-    if (getenv("XTQ_VIT_GROUP")) return n < 4 * ncu;
-    // (beyond, a round is a small part of the whole and T decides)
-    if (n >= 16 * ncu) return false;
-    double rows = 1.5e-6 / 4.7 * (double)xtq::bp_tile_bytes(K) * n;      // us
-    const double lat = 22.0 + 28.0 * (double)xtq::bp_step_bytes(K) / 4096.0;
-    rows = rows < lat ? lat : rows > 300.0 ? 300.0 : rows;
-    const double split =
-        xtq::forward_cost_us(K, xtq::forward_group(K, n, ncu), n, ncu) * (n1 + xtq::kSteps);
-    // steps' time per traceback
-    const int tb1 = K > 2 ? 7 : 2 * n < ncu ? 12 : 25, tb2 = K > 2 ? 16 : 2 * n < ncu ? 26 : 50;
-    return fused_steps(n, n1 + tb1, xtq::kSteps + tb2, ncu) * xtq::forward_step_us(K, 1) <=
-           split + rows + 50.0;
+    if (getenv("XTQ_VIT_GROUP")) return n < 4 * (cx.ncu > 0 ? cx.ncu : 1);
+    return xtq::fused_ends_first(K, xtq::forward_group_max(K), (double)xtq::bp_step_bytes(K), n,
+                                 n1, pivot, xtq::kSteps, cx.ncu);
 }
 
 // Whether the tracebacks of a chunk of n sequences use one lane per
@@ -576,7 +540,7 @@ int tailbite_chunks(DevCtx& cx, const TbScratch& w, int chunk, const float* dX, 
             }
             continue;
         }
-        if (use_fused(cx, K, n, n1)) {
+        if (use_fused(cx, K, n, n1, pivot)) {
             if (++cx.epoch == 0) cx.epoch = 1;
             const int pf = pbeg(0, (double)n * (n1 + xtq::kSteps));
             e = xtq::launch_tailbite_fused(K, x, n, lut, pivot, n1, w.bp, w.ov, w.flags,

@@ -1,0 +1,98 @@
+// route.h -- how a batch of sequences is launched: the sequences per forward
+// workgroup, and the fused two-pass launch or separate ones.  Host code
+// without a device, from times measured on 256 CUs.
+#pragma once
+
+namespace xtq {
+
+// Microseconds one CU takes per step of one sequence, by K and sequences per
+// workgroup (1, 2, 4, 8), measured over tail-bites of 16,384 sequences.
+inline double forward_step_us(int K, int T) {
+    static const double us[6][4] = {{1.350, 1.350, 1.350, 1.350}, {1.258, 1.255, 1.255, 1.255},
+                                    {1.190, 1.219, 1.171, 1.171}, {1.242, 1.235, 1.217, 1.198},
+                                    {1.281, 1.292, 1.235, 1.220}, {1.309, 1.298, 1.261, 1.231}};
+    if (K < 2 || K > 7) return 1.0;
+    return us[K - 2][T <= 1 ? 0 : T <= 2 ? 1 : T <= 4 ? 2 : 3];
+}
+
+// Estimated microseconds per step of a launch of nseq >= 1 sequences, T per
+// workgroup, on ncu CUs: one workgroup per CU is resident, so the launch runs
+// in rounds of ncu workgroups, each T sequences long.
+inline double forward_cost_us(int K, int T, int nseq, int ncu) {
+    if (ncu < 1) ncu = 1;
+    const int wgs = (nseq - 1) / T + 1, rounds = (wgs - 1) / ncu + 1;
+    return (double)rounds * T * forward_step_us(K, T);
+}
+
+// Sequences per workgroup, at most max_T (the LDS bounds it by K), that finish
+// nseq sequences first: a group that fills its last round beats a larger one
+// that does not (K=4, tail-bite calls on 256 CUs: 2000 sequences T = 1 in eight
+// rounds 5.10 ms, T = 4 in two 5.05; 1500 T = 1 in six 3.84, T = 4 in two 4.93).
+inline int forward_group(int K, int max_T, int nseq, int ncu) {
+    int best = 1;
+    double cost = forward_cost_us(K, 1, nseq, ncu);
+    for (int T = 2; T <= max_T; T *= 2) {
+        const double c = forward_cost_us(K, T, nseq, ncu);
+        if (c <= cost) {
+            best = T;
+            cost = c;
+        }
+    }
+    return best;
+}
+
+// Steps until the last of a fused launch's 2 nseq workgroups ends: each CU
+// takes the next of nseq first passes and then of nseq second passes, of d1 and
+// d2 steps, as soon as it is free.
+inline double fused_steps(int nseq, int d1, int d2, int ncu) {
+    const int r = nseq / ncu, m = nseq % ncu;  // pass 1: m CUs take r + 1, the others r
+    const int cus[2] = {ncu - m, m};
+    double t[2] = {(double)r * d1, (double)(r + 1) * d1};
+    double end = m ? t[1] : t[0];
+    for (int left = nseq; left > 0;) {
+        const int g = m && t[1] < t[0] ? 1 : 0;            // the CUs free first
+        t[g] = (t[g] < d1 ? d1 : t[g]) + d2;               // (a pass 2 waits for its pass 1)
+        if (t[g] > end) end = t[g];
+        left -= cus[g];
+    }
+    return end;
+}
+
+// Whether a tail-bite of nseq sequences (n1 steps of pass 1, its pivot, nsteps
+// of pass 2, row_bytes of backpointers per step) ends sooner as one fused
+// launch than as separate ones.
+//   The fused launch fills its rounds with 2 nseq passes of one sequence, each
+// with its own traceback: 26 (K=7) to 40 steps' time (K=2), half of what a pair
+// of passes takes beyond 512 steps at 16,384 sequences.  Separate launches run
+// T sequences per workgroup and read the kept rows again, at 4.7 TB/s, or in
+// 0.3 ms with one lane per sequence.  The fused estimate is raised by 1.5 %:
+// with that the choices lose least against the faster route, 0.1 % on average
+// and 4 % at most over 540 batches of 1 to 6000 sequences (K = 2..7, three
+// pivots, two devices), which is as far as two runs of one batch differ.
+//   Up to one sequence per CU both take two rounds at best and the separate
+// launches are the sooner (192 sequences fused even take the time of three: the
+// second passes that start early wait on CUs, presumably unevenly over the
+// dies, to which workgroups are dealt in turn).  From 16 per CU a round is a
+// small part of the whole.
+//   Whole calls, pivot 128, fused / separate, us.  K=4: 1 sequence 640 / 636,
+// 64 713 / 670, 192 1087 / 700, 256 804 / 708; 257 1084 / 1273, 300 1080 / 1259,
+// 400 1422 / 1258, 513 1765 / 1828, 600 1752 / 1873, 768 2105 / 1960, 1003
+// 2737 / 2507, 1025 3058 / 3061, 2049 5844 / 5622.  K=2: 1 734 / 738, 64 789 /
+// 754, 128 840 / 765, 300 1185 / 1435, 512 1599 / 1559, 513 1943 / 2138, 1003
+// 3135 / 3094, 1025 3539 / 3693, 1537 5094 / 5199, 2049 6752 / 6451.  K=7: 64
+// 787 / 736, 300 1217 / 1378, 600 2007 / 2055, 1003 3036 / 2668.
+inline bool fused_ends_first(int K, int max_T, double row_bytes, int nseq, int n1, int pivot,
+                             int nsteps, int ncu) {
+    if (K < 2 || K > 7) return false;
+    if (ncu < 1) ncu = 1;
+    if (nseq <= ncu || nseq >= 16 * ncu) return false;
+    static const int tb[6] = {40, 39, 35, 28, 31, 26};
+    const double fused = 1.015 * forward_step_us(K, 1) *
+                         fused_steps(nseq, n1 + tb[K - 2], nsteps + tb[K - 2], ncu);
+    double rows = row_bytes * nseq * (n1 - 1 - pivot + nsteps - 1) / 4.7e6;        // us
+    if (rows > 300.0) rows = 300.0;
+    const int T = forward_group(K, max_T, nseq, ncu);
+    return fused < forward_cost_us(K, T, nseq, ncu) * (n1 + nsteps) + rows;
+}
+
+}  // namespace xtq

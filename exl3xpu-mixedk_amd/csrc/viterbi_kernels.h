@@ -27,14 +27,8 @@ size_t bp_step_bytes(int K);
 // Bytes of backpointer scratch one sequence needs for a whole pass.
 inline size_t bp_tile_bytes(int K) { return (size_t)kSlots * bp_step_bytes(K); }
 
-// Sequences per forward workgroup: the largest whose LDS fits at K, and the
-// one that finishes nseq >= 1 sequences first on ncu compute units.
+// Sequences per forward workgroup: the most whose LDS fits at K.
 int forward_group_max(int K);
-int forward_group(int K, int nseq, int ncu);
-// Estimated microseconds per trellis step of a launch of nseq >= 1 sequences,
-// T per workgroup, and those of one sequence alone on a CU.
-double forward_cost_us(int K, int T, int nseq, int ncu);
-double forward_step_us(int K, int T);
 
 // Forward DP of one Viterbi run for nseq sequences.
 //   X, xstride, xlen  targets: row q holds xlen fp32 values at X + q*xstride

@@ -1966,39 +1966,6 @@ int forward_group_max(int K) {
     return T;
 }
 
-// Microseconds one CU takes per step of one sequence, by K and sequences per
-// workgroup (1, 2, 4, 8), measured over tail-bites of 16,384 sequences.
-double forward_step_us(int K, int T) {
-    static const double us[6][4] = {{1.390, 1.390, 1.390, 1.390}, {1.447, 1.249, 1.249, 1.249},
-                                    {1.330, 1.209, 1.171, 1.171}, {1.379, 1.235, 1.207, 1.206},
-                                    {1.346, 1.292, 1.234, 1.216}, {1.399, 1.299, 1.271, 1.234}};
-    if (K < 2 || K > 7) return 1.0;
-    return us[K - 2][T <= 1 ? 0 : T <= 2 ? 1 : T <= 4 ? 2 : 3];
-}
-
-// One workgroup per CU is resident, so a launch runs in rounds of ncu
-// workgroups, each round T sequences long: a group that fills its last round
-// beats a larger one that does not (2001 sequences at K=4 on 256 CUs: 8
-// sequence-steps per CU either way, T = 2 in four rounds 5.34, T = 4 in two
-// 5.06 ms; 1500: T = 2 in three rounds 4.07, T = 4 in two 4.94 ms).
-int forward_group(int K, int nseq, int ncu) {
-    int best = 1;
-    double cost = 0.0;
-    for (int T = 1; T <= forward_group_max(K); T *= 2) {
-        const double c = forward_cost_us(K, T, nseq, ncu);
-        if (T == 1 || c <= cost) {
-            best = T;
-            cost = c;
-        }
-    }
-    return best;
-}
-
-double forward_cost_us(int K, int T, int nseq, int ncu) {
-    const int wgs = (nseq - 1) / T + 1, rounds = (wgs - 1) / ncu + 1;
-    return (double)rounds * T * forward_step_us(K, T);
-}
-
 hipError_t launch_forward(int K, const float* X, int xstride, int xlen, int nseq,
                           const float* lut, int roll, int nsteps, int store_lo,
                           const int32_t* ov_in, void* bp, int32_t* send, uint32_t* err,

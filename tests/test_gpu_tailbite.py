@@ -203,14 +203,14 @@ def test_lane_traceback_vs_oracle(hb, oracle_mod, mul1_lut, K, monkeypatch):
 
 @pytest.mark.parametrize("K,n", [(4, 320), (6, 320), (5, 384), (7, 64), (2, 257)])
 def test_fused_ldlq_sized_batches(hb, oracle_mod, mul1_lut, K, n, monkeypatch):
-    """Batch sizes of the BlockLDLQ sweep's launches (one 16-row block: tn
-    tiles), where the fused two-pass launch runs by default: identical to
-    the separate-launch path and to the oracle."""
+    """The fused two-pass launch on batches around one sequence per CU (one
+    16-row block of a BlockLDLQ sweep): identical to the separate-launch path
+    and to the oracle."""
     rng = np.random.default_rng(300 + K)
     X = rng.standard_normal((n, 256)).astype(np.float32)
     X[::7] = mul1_lut[rng.integers(0, 65536, (len(X[::7]), 256))]
     print(f"case fused K={K} n={n}", flush=True)
-    monkeypatch.delenv("XTQ_VIT_FUSED", raising=False)
+    monkeypatch.setenv("XTQ_VIT_FUSED", "1")
     fused, tr = _run(hb, X, K, 128, 0, trellis=True)
     monkeypatch.setenv("XTQ_VIT_FUSED", "0")
     split, _ = _run(hb, X, K, 128, 0)
@@ -288,7 +288,7 @@ def test_forced_chunks(hb, oracle_mod, mul1_lut, K, monkeypatch):
     """XTQ_VIT_SCRATCH is read on every call: a budget of 2048 sequences
     splits a batch of 2 x 2048 + 700 into three chunks with a partial last
     one (the full chunks take the separate-pass path with one-lane
-    tracebacks, the last the fused path).  Every tile equals the unchunked
+    tracebacks, the last the path that is estimated to end first).  Every tile equals the unchunked
     run, and the first and last 32 tiles of each chunk equal the oracle."""
     per = hb.scratch_per_seq(K)
     rnd = 4 * torch.cuda.get_device_properties(0).multi_processor_count
@@ -333,7 +333,9 @@ def test_decode_unpack_pack(hb, oracle_mod, mul1_lut, K):
     np.testing.assert_array_equal(w.cpu().numpy(), oracle_mod.decode(rnd, mul1_lut, K))
 
 
-def test_nan_target_rejected(hb):
+@pytest.mark.parametrize("fused", ("0", "1"))
+def test_nan_target_rejected(hb, fused, monkeypatch):
+    monkeypatch.setenv("XTQ_VIT_FUSED", fused)
     X = torch.randn(3, 256, device="cuda")
     X[1, 17] = float("nan")
     with pytest.raises(hb.HipViterbiError) as ei:
