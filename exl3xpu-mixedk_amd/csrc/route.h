@@ -16,12 +16,27 @@ inline double forward_step_us(int K, int T) {
 }
 
 // Estimated microseconds per step of a launch of nseq >= 1 sequences, T per
-// workgroup, on ncu CUs: one workgroup per CU is resident, so the launch runs
-// in rounds of ncu workgroups, each T sequences long.
+// workgroup, on ncu CUs.  One workgroup per CU is resident, so the launch runs
+// in rounds of ncu workgroups, each T sequences long.  The last workgroup takes
+// the nseq % T sequences that are left, and where the others fill whole rounds
+// it is a round by itself: of its own length, not of T sequences (K=4, T = 4 on
+// 256 CUs, us a step: 1024 / 1025 / 1026 / 1028 sequences 4.60 / 6.02 / 7.35 /
+// 9.20).  It has its CU to itself without enough sequences to cover each
+// other's latency, which takes it 1.2 times the one-sequence time for each (1.43
+// to 1.57 us alone, two 2.7 to 2.9, four of eight 5.2 to 5.6), up to a whole
+// workgroup's.
 inline double forward_cost_us(int K, int T, int nseq, int ncu) {
     if (ncu < 1) ncu = 1;
-    const int wgs = (nseq - 1) / T + 1, rounds = (wgs - 1) / ncu + 1;
-    return (double)rounds * T * forward_step_us(K, T);
+    const int full = nseq / T, rest = nseq % T;
+    const double round = T * forward_step_us(K, T);
+    double us = (double)(full / ncu) * round;
+    if (full % ncu) {
+        us += round;
+    } else if (rest) {
+        const double own = 1.2 * rest * forward_step_us(K, 1);
+        us += own < round ? own : round;
+    }
+    return us;
 }
 
 // Sequences per workgroup, at most max_T (the LDS bounds it by K), that finish

@@ -1,5 +1,7 @@
-"""How a batch is launched (csrc/route.h), compiled for the host, against
-measured times."""
+"""How a batch is launched (csrc/route.h), compiled for the host: the estimate
+of a launch's time against its workgroups taken one by one, and the choices
+against measured times."""
+import heapq
 import os
 import subprocess
 
@@ -45,6 +47,51 @@ def route(tmp_path_factory):
         return [float(v) for v in out.split()]
 
     return ask
+
+
+@pytest.mark.parametrize("K", range(2, 8))
+def test_cost_is_the_end_of_the_last_workgroup(route, K):
+    """Each CU takes the next workgroup as soon as it is free.  A last one of
+    fewer than T sequences is shorter than the others, so it never costs a
+    round of T sequences."""
+    for ncu in (1, 5, NCU):
+        for T in [t for t in (1, 2, 4, 8) if t <= MAX_T[K]]:
+            us1, us = route([("s", K, 1, 0, 0), ("s", K, T, 0, 0)])
+            ns = sorted({n for r in (1, 2, 3) for n in range(r * T * ncu - T, r * T * ncu + 2 * T)
+                         if n > 0} | {1, 2, 3, 7, 100})
+            got = route([("c", K, T, n, ncu) for n in ns])
+            for n, g in zip(ns, got):
+                cus = [0.0] * ncu
+                for q in range(0, n, T):
+                    r = min(T, n - q)
+                    t = T * us if r == T else min(T * us, 1.2 * r * us1)
+                    heapq.heappush(cus, heapq.heappop(cus) + t)
+                assert g == pytest.approx(max(cus), rel=1e-12), (K, T, n, ncu)
+
+
+# Microseconds per step of the forwards of a tail-bite of n sequences on 256
+# CUs, by sequences per workgroup (1, 2, 4, 8).
+MEASURED = {
+    (3, 513): (3.574, 3.781), (3, 1025): (5.960, 6.247), (3, 2049): (10.872, 11.184),
+    (4, 257): (2.370, 2.423, 4.455), (4, 513): (3.382, 3.825, 4.437),
+    (4, 1025): (5.667, 6.247, 6.016), (4, 1026): (5.706, 7.187, 7.351),
+    (4, 1537): (7.960, 8.666, 9.221), (4, 2049): (10.470, 11.129, 10.702),
+    (4, 2053): (10.662, 12.449, 14.340),
+    (5, 1025): (5.790, 6.249, 5.992, 8.767), (5, 2049): (10.833, 11.265, 10.808, 10.850),
+    (5, 2053): (10.864, 12.636, 14.502, 16.960), (5, 3073): (15.806, 16.618, 15.945, 18.855),
+    (6, 1025): (6.215, 6.661, 6.392, 9.413), (6, 2049): (11.417, 11.854, 11.421, 11.225),
+    (7, 1025): (6.430, 6.729, 6.615, 9.560), (7, 2049): (11.725, 11.997, 11.721, 11.321),
+    (7, 2048): (10.482, 10.457, 10.090, 9.842), (7, 3073): (16.990, 17.195, 16.964, 19.912),
+}
+
+
+def test_group_choice_against_measured_times(route):
+    """Around whole rounds, where a larger group's last workgroup may be short:
+    the chosen group's time is the least measured, within the 3.5 % by which
+    two runs of one size differ here."""
+    got = route([("g", K, MAX_T[K], n, NCU) for K, n in MEASURED])
+    for (key, us), T in zip(MEASURED.items(), got):
+        assert us[int(T).bit_length() - 1] <= 1.035 * min(us), (key, T)
 
 
 # Microseconds of whole tail-bite calls on 256 CUs, (K, sequences, pivot,
