@@ -171,8 +171,9 @@ def had_right(w: torch.Tensor, h: torch.Tensor) -> torch.Tensor:
 
 def _fold_scales(w: torch.Tensor, suh: torch.Tensor, svh: torch.Tensor) -> bool:
     """Whether the kernels apply the channel scales in the transforms' passes:
-    fp32 GPU weights with one scale per row and per column there.  Anything
-    else takes the separate torch passes below."""
+    fp32 GPU weights (of any strides) with one scale per row and per column
+    there (of any type, taken as fp32).  Anything else takes the separate torch
+    passes below."""
     return (w.is_cuda and w.dtype == torch.float32 and w.dim() == 2
             and w.shape[0] % 128 == 0 and w.shape[1] % 128 == 0
             and suh.shape == w.shape[:1] and svh.shape == w.shape[1:]
@@ -190,10 +191,20 @@ def to_inner(w_orig: torch.Tensor, suh: torch.Tensor, svh: torch.Tensor,
     return had_right(had_left(w, h), h)
 
 
+def _differentiated(t: torch.Tensor) -> bool:
+    """Whether torch follows t through its own operations: for a gradient, a
+    forward-mode tangent, or a batch (vmap)."""
+    return (torch._C._functorch.is_functorch_wrapped_tensor(t)
+            or (t.requires_grad and torch.is_grad_enabled())
+            or torch.autograd.forward_ad.unpack_dual(t).tangent is not None)
+
+
 def from_inner(w_inner: torch.Tensor, suh: torch.Tensor, svh: torch.Tensor,
                h: torch.Tensor) -> torch.Tensor:
-    """W_inner -> W_orig = diag(suh) B_k W_i B_n diag(svh)."""
-    if _fold_scales(w_inner, suh, svh):
+    """W_inner -> W_orig = diag(suh) B_k W_i B_n diag(svh).  The product with
+    svh is torch's own where torch has to see it (the result is linear in it);
+    the transforms are not differentiable."""
+    if _fold_scales(w_inner, suh, svh) and not _differentiated(svh):
         return _hb.had128_both(w_inner.contiguous(), h.to(w_inner.device, torch.float32),
                                suh.float(), svh.float(), divide=False)
     w = had_left(w_inner, h) * suh.float().unsqueeze(1)

@@ -32,6 +32,34 @@ def test_scaled_transforms_match_cpu(xq, k, n):
     assert torch.equal(xq.to_inner(w.cuda(), sud.double(), svd.double(), hd).cpu(), want_in)
 
 
+def test_from_inner_follows_column_scales(xq):
+    """from_inner's product with the column scales stays torch's where torch
+    follows them: a gradient, a tangent and a batch of scales equal the CPU's."""
+    g = torch.Generator().manual_seed(5)
+    w = torch.randn(128, 256, generator=g)
+    su = torch.randn(128, generator=g) + 3.0
+    sv = torch.randn(256, generator=g) + 3.0
+    svs = torch.randn(3, 256, generator=g) + 3.0
+    h = xq.hadamard128(None, torch.float32)
+    res = {}
+    for dev in ("cpu", "cuda"):
+        a = [t.to(dev) for t in (w, su, sv, svs, h)]
+        v = a[2].clone().requires_grad_()
+        out = xq.from_inner(a[0], a[1], v, a[4])
+        assert out.requires_grad
+        # one term per column: no sum whose order could differ
+        grad, = torch.autograd.grad(out[7].sum(), v)
+        with torch.autograd.forward_ad.dual_level():
+            dual = torch.autograd.forward_ad.make_dual(a[2], a[3][0])
+            tan = torch.autograd.forward_ad.unpack_dual(xq.from_inner(a[0], a[1], dual, a[4]))[1]
+        batch = torch.vmap(lambda s: xq.from_inner(a[0], a[1], s, a[4]))(a[3])
+        with torch.no_grad():
+            assert not xq.from_inner(a[0], a[1], v, a[4]).requires_grad
+        res[dev] = [t.detach().cpu() for t in (out, grad, tan, batch)]
+    for got, want in zip(res["cuda"], res["cpu"]):
+        assert torch.equal(got, want)
+
+
 def test_scaled_transforms_more_blocks_than_workgroups(xq):
     """17 x 17 blocks (a second round for 33 of the 256 workgroups) and
     multipliers that are not symmetric."""
