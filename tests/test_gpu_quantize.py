@@ -277,8 +277,8 @@ def test_hadamard_kernel_matches_cpu(xq, k, n):
 
 @pytest.mark.parametrize("rows", [1, 7, 37, 1000])
 def test_had_right_ragged_rows(xq, rows):
-    """had_right on the GPU for row counts that leave a partial wave (the
-    kernel takes 8 rows per wave): each output row depends on its own input
+    """had_right on the GPU for row counts that leave a partial tile (the
+    kernel takes 64 rows at a time): each output row depends on its own input
     row only, so the rows of the CPU product of a 1024-row matrix are the
     reference (a shape whose CPU sgemm is one FMA chain per output)."""
     g = torch.Generator().manual_seed(rows)
