@@ -152,6 +152,7 @@ static __device__ __align__(256) uint8_t scratch[kNoAllocBytes];
 
 // Opt-in kernel timing: each forward/traceback launch is bracketed with HIP
 // events on its stream; elapsed times are folded in after the stream syncs.
+// Launches with their tracebacks inside are of the forward kind.
 struct ProfPair { hipEvent_t a, b; int kind; double seq_steps; };
 bool g_prof = false;
 std::vector<ProfPair> g_prof_pending;
@@ -1171,8 +1172,6 @@ int xtq_trellis_decode_dev(const int16_t* d_trellis, int tk, int tn, int K, cons
     if (rc) return rc;
     int dev = 0;
     if (current_device(&dev)) return 1;
-    rc = dev_init(dev);
-    if (rc) return rc;
     hipError_t e = xtq::launch_decode(K, (int)c, d_trellis, tk, tn, d_out_f32, d_out_f16,
                                       (hipStream_t)stream);
     if (e != hipSuccess) {
@@ -1215,6 +1214,7 @@ int xtq_had128_right_dev(const float* d_h, const float* d_in, float* d_out, int 
                          void* stream) {
     if (!d_h || !d_in || !d_out) return 12;
     if (d_in == d_out) return 12;
+    // (the documented maximum; the kernel's own limit is higher)
     if (rows <= 0 || cols <= 0 || cols % 128 || (rows + 31) / 32 > 65535) return 6;
     return had_status(
         xtq::launch_had_right(d_h, d_in, d_out, rows, cols, (hipStream_t)stream));
@@ -1225,6 +1225,7 @@ int xtq_had128_both_dev(const float* d_h, const float* d_in, float* d_out, int r
                         void* stream) {
     if (!d_h || !d_in || !d_out || !d_row_scale || !d_col_scale) return 12;
     if (d_in == d_out) return 12;
+    // (what the two transforms take one after the other)
     if (rows <= 0 || cols <= 0 || rows % 128 || cols % 128 || (rows + 31) / 32 > 65535) return 6;
     return had_status(xtq::launch_had_both(d_h, d_in, d_out, rows, cols, d_row_scale, d_col_scale,
                                            divide != 0, (hipStream_t)stream));
