@@ -470,7 +470,8 @@ def _roofline_fields(tiles: int, dt: float, prof: dict) -> dict:
         f["encode_kernel_frac"] = round(kops / FP32_PEAK, 4)
         f["encode_kernel_note"] = ("column-chain launch (feedback, both passes, tracebacks and "
                                    "outputs of every tile)" if xq.DEFAULT_SCHEDULE != "block"
-                                   else "forward launches of the block schedule")
+                                   else "forward launches of the block schedule (fused ones "
+                                        "with their tracebacks)")
     return f
 
 

@@ -4,8 +4,9 @@
 // A tile is a 256 K-bit stream of 8K 32-bit words, MSB first: symbol t
 // (s_t mod 2^K) at bits [tK, (t+1)K), and state t the 16-bit circular window
 // that ends with symbol t's bits.  All three kernels move bytes: what bounds
-// them is HBM, and their work is arranged so that every lane's accesses are
-// 16 bytes and a wave's are contiguous.
+// them is HBM, and their work is arranged so that a lane's fp32 values and
+// states move 16 bytes at a time (fp16 values 8) and a wave's are contiguous.
+// The trellis, a fifth of the bytes at most, moves in its 4-byte words.
 #include "viterbi_kernels.h"
 
 #pragma clang fp contract(off)
@@ -14,7 +15,7 @@ namespace xtq {
 namespace {
 
 // Global-memory vectors of the callers' alignment (the element's own): the
-// accesses are 16 bytes wide all the same, gfx950 takes them at any address.
+// accesses are as wide all the same, gfx950 takes them at any address.
 typedef uint32_t u32_t __attribute__((aligned(2)));
 typedef float f32x4_t __attribute__((ext_vector_type(4), aligned(4)));
 typedef _Float16 f16x4_t __attribute__((ext_vector_type(4), aligned(2)));
@@ -28,7 +29,8 @@ __device__ __forceinline__ uint32_t window(uint32_t hi, uint32_t lo, uint32_t sh
 
 // Codebook value of state s, bit for bit the table's (quantize.py:56-87).
 // Computed instead of looked up: 89 M lookups in the 256 KiB table go to L2,
-// and took 0.45 ms of a 17408x5120 decode; these are 4 to 12 instructions.
+// and took 0.45 ms of a 17408x5120 decode; these take a handful of
+// instructions, 1mad's with those of a correctly rounded division.
 //   mul1   (1024 + byte sum) c1 + c2 with c1 = 1774/2^18, c2 = -1329/2^7: every
 //          term and the sum fit 24 bits, so the fp32 value is exact and only
 //          the rounding to fp16 remains, as in the reference's fp64

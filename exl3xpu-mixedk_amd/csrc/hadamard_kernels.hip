@@ -29,8 +29,10 @@ typedef float v32f __attribute__((ext_vector_type(32)));
 typedef float f32x4_t __attribute__((ext_vector_type(4), aligned(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 
-constexpr int kHadGroups = 512;        // workgroups of a launch: two per CU
-constexpr int kHadBothGroups = 256;    // of had_both: one per CU
+// Most workgroups of a launch, two (had_both: one) for each of the MI355X's 256
+// CUs; they take the tiles in turn, so any number of CUs is right.
+constexpr int kHadGroups = 512;
+constexpr int kHadBothGroups = 256;
 
 // Row of accumulator register v in its 32x32 block, for the lane's half.
 __device__ __forceinline__ int acc_row(int v, int ln) {

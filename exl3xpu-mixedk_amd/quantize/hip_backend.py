@@ -405,7 +405,8 @@ def prof_enable(on: bool = True):
 
 def prof_read() -> dict:
     """Totals since the last read: forward ms/launches/sequence-steps and
-    traceback ms/launches (xtq_vit_prof_read)."""
+    traceback ms/launches (xtq_vit_prof_read; fused launches and column chains
+    count whole as forward)."""
     fm, ss, tm = ctypes.c_double(), ctypes.c_double(), ctypes.c_double()
     fl, tl = ctypes.c_int64(), ctypes.c_int64()
     lib().xtq_vit_prof_read(ctypes.byref(fm), ctypes.byref(fl), ctypes.byref(ss),

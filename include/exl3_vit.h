@@ -61,7 +61,8 @@
  *   XTQ_VIT_GROUP    force 1, 2, 4 or 8 sequences per forward workgroup
  *                    (testing; default chosen from the batch size)
  *   XTQ_VIT_TB_LANES smallest batch whose tracebacks run one lane per sequence
- *                    (0: always, -1: never; default 2048)
+ *                    (0: always, -1: never; default 2048); fused launches
+ *                    trace back inside and do not ask
  *   XTQ_VIT_FUSED    0: always run the two tail-biting passes as separate
  *                    launches; 1: always as one fused launch (testing);
  *                    default: whichever is estimated to end first
@@ -331,6 +332,9 @@ XTQ_API int xtq_vit_chunk_seqs(int nseq, int K, int* deferred);
  * on the stream it runs on.  xtq_vit_prof_read returns and resets the totals:
  * forward milliseconds, forward launches, forward sequence-steps (sum of
  * sequences x steps over the launches), traceback milliseconds and launches.
+ * A launch with its tracebacks inside (a fused tail-bite, a column chain)
+ * counts whole as one forward launch and as no traceback.  Single Viterbi runs
+ * are not timed.
  */
 XTQ_API int xtq_vit_prof_enable(int on);
 XTQ_API int xtq_vit_prof_read(double* fwd_ms, int64_t* fwd_launches, double* fwd_seq_steps,
