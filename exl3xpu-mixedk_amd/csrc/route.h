@@ -82,25 +82,34 @@ inline double fused_steps(int nseq, int d1, int d2, int ncu) {
 // T sequences per workgroup and read the kept rows again, at 4.7 TB/s, or in
 // 0.3 ms with one lane per sequence.  The fused estimate is raised by 1.5 %:
 // with that the choices lose least against the faster route, 0.1 % on average
-// and 4 % at most over 540 batches of 1 to 6000 sequences (K = 2..7, three
+// and 4 % at most over 474 batches of 257 to 6000 sequences (K = 2..7, three
 // pivots, two devices), which is as far as two runs of one batch differ.
-//   Up to one sequence per CU both take two rounds at best and the separate
-// launches are the sooner (192 sequences fused even take the time of three: the
-// second passes that start early wait on CUs, presumably unevenly over the
-// dies, to which workgroups are dealt in turn).  From 16 per CU a round is a
-// small part of the whole.
-//   Whole calls, pivot 128, fused / separate, us.  K=4: 1 sequence 640 / 636,
-// 64 713 / 670, 192 1087 / 700, 256 804 / 708; 257 1084 / 1273, 300 1080 / 1259,
-// 400 1422 / 1258, 513 1765 / 1828, 600 1752 / 1873, 768 2105 / 1960, 1003
-// 2737 / 2507, 1025 3058 / 3061, 2049 5844 / 5622.  K=2: 1 734 / 738, 64 789 /
-// 754, 128 840 / 765, 300 1185 / 1435, 512 1599 / 1559, 513 1943 / 2138, 1003
-// 3135 / 3094, 1025 3539 / 3693, 1537 5094 / 5199, 2049 6752 / 6451.  K=7: 64
-// 787 / 736, 300 1217 / 1378, 600 2007 / 2055, 1003 3036 / 2668.
+//   Up to one sequence per CU both take two rounds at best.  On the GPU the
+// separate launches are the sooner from some 40 sequences on: a fused launch's
+// waiting workgroups poll, and where its 2 nseq are not all resident (above half
+// a sequence per CU) second passes that start early hold CUs, presumably
+// unevenly over the dies to which workgroups are dealt in turn, and the time is
+// that of three rounds.  Between other kernels, as in quantize_seq_tailbite,
+// four launches take some 20 us longer than back to back and one launch does
+// not: there the two cross at 80 to 90 sequences of 256 CUs, where the line is.
+// From 16 sequences per CU a round is a small part of the whole.
+//   quantize_seq_tailbite, pivot 128, fused / separate, us.  K=4: 1 sequence
+// 671 / 669, 8 682 / 728, 64 729 / 734, 80 737 / 746, 96 763 / 738, 128 756 /
+// 731, 192 1061 / 740, 256 768 / 743, 300 1096 / 1316, 400 1421 / 1326, 513
+// 1768 / 1909, 600 1778 / 1943, 1003 2804 / 2578.  K=2: 8 771 / 828, 64 823 /
+// 837, 96 854 / 832, 128 845 / 856, 192 1195 / 850, 256 859 / 857, 300 1240 /
+// 1528, 400 1642 / 1548, 513 2004 / 2225, 1003 3189 / 3145.  K=7: 8 744 / 783,
+// 64 792 / 812, 80 800 / 847, 96 809 / 809, 128 838 / 811, 192 1162 / 817, 300
+// 1180 / 1495, 600 1915 / 2138, 1003 3014 / 2732.
+//   The library's own entry, K=4: 64 713 / 670, 768 2105 / 1960, 1025 3058 /
+// 3061, 2049 5844 / 5622; K=2: 512 1599 / 1559, 1025 3539 / 3693, 1537 5094 /
+// 5199.
 inline bool fused_ends_first(int K, int max_T, double row_bytes, int nseq, int n1, int pivot,
                              int nsteps, int ncu) {
     if (K < 2 || K > 7) return false;
     if (ncu < 1) ncu = 1;
-    if (nseq <= ncu || nseq >= 16 * ncu) return false;
+    if (nseq <= ncu) return 3 * nseq <= ncu;
+    if (nseq >= 16 * ncu) return false;
     static const int tb[6] = {40, 39, 35, 28, 31, 26};
     const double fused = 1.015 * forward_step_us(K, 1) *
                          fused_steps(nseq, n1 + tb[K - 2], nsteps + tb[K - 2], ncu);

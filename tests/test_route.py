@@ -97,36 +97,53 @@ def test_group_choice_against_measured_times(route):
 # Microseconds of whole tail-bite calls on 256 CUs, (K, sequences, pivot,
 # margin): as separate launches at the best group, and as one fused launch.
 ROUTES = {
-    (2, 64, 128, 0): (754, 789), (2, 128, 128, 0): (765, 840), (2, 192, 128, 0): (780, 1186),
-    (2, 257, 128, 0): (1401, 1168), (2, 300, 128, 0): (1435, 1185), (2, 400, 128, 0): (1466, 1571),
-    (2, 512, 128, 0): (1559, 1599), (2, 513, 128, 0): (2138, 1943), (2, 600, 128, 0): (2221, 1977),
-    (2, 1003, 128, 0): (3094, 3135), (2, 1025, 128, 0): (3693, 3539),
-    (2, 1537, 128, 0): (5199, 5094), (2, 2049, 128, 0): (6451, 6752), (2, 64, 128, 16): (579, 628),
-    (2, 257, 128, 16): (1094, 1018), (2, 600, 128, 16): (1720, 1637), (3, 64, 128, 0): (712, 751),
-    (3, 256, 128, 0): (790, 815), (3, 257, 128, 0): (1318, 1136), (3, 300, 128, 0): (1343, 1141),
-    (3, 400, 128, 0): (1374, 1497), (3, 513, 128, 0): (2016, 1850), (3, 600, 128, 0): (2073, 1856),
-    (3, 768, 128, 0): (2180, 2237), (3, 1003, 128, 0): (2851, 2943),
-    (3, 1200, 128, 0): (3554, 3693), (3, 1500, 128, 0): (4271, 4447),
-    (3, 2300, 128, 0): (6027, 6769), (4, 64, 128, 0): (670, 713), (4, 256, 128, 0): (708, 804),
-    (4, 257, 128, 0): (1273, 1084), (4, 300, 128, 0): (1259, 1080), (4, 400, 128, 0): (1258, 1422),
-    (4, 513, 128, 0): (1828, 1765), (4, 600, 128, 0): (1873, 1752), (4, 768, 128, 0): (1960, 2105),
-    (4, 1003, 128, 0): (2507, 2737), (4, 1200, 128, 0): (3189, 3436),
-    (4, 1500, 128, 0): (3836, 4177), (4, 2300, 128, 0): (5746, 6266), (5, 64, 128, 0): (676, 721),
-    (5, 256, 128, 0): (746, 844), (5, 257, 128, 0): (1310, 1128), (5, 300, 128, 0): (1283, 1151),
-    (5, 400, 128, 0): (1314, 1511), (5, 513, 128, 0): (1881, 1871), (5, 600, 128, 0): (1916, 1880),
-    (5, 768, 128, 0): (2050, 2249), (5, 1003, 128, 0): (2529, 2837),
+    (2, 1, 128, 0): (785, 763), (2, 1, 128, 16): (605, 602), (2, 8, 128, 0): (828, 771),
+    (2, 8, 128, 16): (664, 619), (2, 64, 128, 0): (837, 823), (2, 64, 128, 16): (667, 652),
+    (2, 128, 128, 0): (856, 845), (2, 128, 128, 16): (671, 704), (2, 192, 128, 0): (850, 1195),
+    (2, 192, 128, 16): (680, 1059), (2, 256, 128, 0): (857, 859), (2, 256, 128, 16): (681, 705),
+    (2, 257, 128, 0): (1401, 1168), (2, 257, 128, 16): (1094, 1018),
+    (2, 300, 128, 0): (1528, 1240), (2, 300, 128, 16): (1195, 1078),
+    (2, 400, 128, 0): (1548, 1642), (2, 400, 128, 16): (1218, 1449),
+    (2, 512, 128, 0): (1559, 1599), (2, 513, 128, 0): (2225, 2004),
+    (2, 513, 128, 16): (1797, 1686), (2, 600, 128, 0): (2334, 2029),
+    (2, 600, 128, 16): (1810, 1702), (2, 1003, 128, 0): (3145, 3189),
+    (2, 1003, 128, 16): (2607, 2700), (2, 1025, 128, 0): (3693, 3539),
+    (2, 1537, 128, 0): (5199, 5094), (2, 2049, 128, 0): (6451, 6752), (3, 1, 128, 0): (716, 709),
+    (3, 8, 128, 0): (763, 724), (3, 64, 128, 0): (785, 774), (3, 128, 128, 0): (779, 803),
+    (3, 192, 128, 0): (795, 1172), (3, 256, 128, 0): (818, 832), (3, 257, 128, 0): (1318, 1136),
+    (3, 300, 128, 0): (1468, 1194), (3, 400, 128, 0): (1498, 1541), (3, 513, 128, 0): (2115, 1917),
+    (3, 600, 128, 0): (2163, 1906), (3, 768, 128, 0): (2180, 2237),
+    (3, 1003, 128, 0): (2996, 3009), (3, 1200, 128, 0): (3554, 3693),
+    (3, 1500, 128, 0): (4271, 4447), (3, 2300, 128, 0): (6027, 6769), (4, 1, 128, 0): (669, 671),
+    (4, 8, 128, 0): (728, 682), (4, 64, 128, 0): (734, 729), (4, 128, 128, 0): (731, 756),
+    (4, 192, 128, 0): (740, 1061), (4, 256, 128, 0): (743, 768), (4, 257, 128, 0): (1273, 1084),
+    (4, 300, 128, 0): (1316, 1096), (4, 400, 128, 0): (1326, 1421), (4, 513, 128, 0): (1909, 1768),
+    (4, 600, 128, 0): (1943, 1778), (4, 768, 128, 0): (1960, 2105),
+    (4, 1003, 128, 0): (2578, 2804), (4, 1200, 128, 0): (3189, 3436),
+    (4, 1500, 128, 0): (3836, 4177), (4, 2300, 128, 0): (5746, 6266), (5, 1, 128, 0): (690, 680),
+    (5, 1, 128, 16): (545, 536), (5, 8, 128, 0): (752, 694), (5, 8, 128, 16): (598, 553),
+    (5, 64, 128, 0): (751, 750), (5, 64, 128, 16): (626, 595), (5, 128, 128, 0): (754, 786),
+    (5, 128, 128, 16): (615, 641), (5, 192, 128, 0): (756, 1097), (5, 192, 128, 16): (613, 925),
+    (5, 256, 128, 0): (759, 802), (5, 256, 128, 16): (623, 642), (5, 257, 128, 0): (1310, 1128),
+    (5, 300, 128, 0): (1432, 1114), (5, 300, 128, 16): (1102, 947), (5, 400, 128, 0): (1403, 1470),
+    (5, 400, 128, 16): (1096, 1283), (5, 513, 128, 0): (1960, 1792),
+    (5, 513, 128, 16): (1573, 1509), (5, 600, 128, 0): (2001, 1810),
+    (5, 600, 128, 16): (1579, 1512), (5, 768, 128, 0): (2050, 2249),
+    (5, 1003, 128, 0): (2615, 2863), (5, 1003, 128, 16): (2035, 2408),
     (5, 1200, 128, 0): (3282, 3556), (5, 1500, 128, 0): (3945, 4242),
-    (5, 2300, 128, 0): (5923, 6507), (6, 64, 128, 0): (707, 763), (6, 256, 128, 0): (771, 877),
-    (6, 257, 128, 0): (1378, 1187), (6, 300, 128, 0): (1355, 1183), (6, 400, 128, 0): (1361, 1577),
-    (6, 513, 128, 0): (1972, 1944), (6, 600, 128, 0): (2003, 1933), (6, 768, 128, 0): (2097, 2299),
-    (6, 1003, 128, 0): (2633, 2959), (6, 1200, 128, 0): (3365, 3694),
-    (6, 1500, 128, 0): (4053, 4449), (6, 2300, 128, 0): (6180, 6767), (7, 64, 128, 0): (736, 787),
-    (7, 256, 128, 0): (784, 902), (7, 257, 128, 0): (1386, 1197), (7, 300, 128, 0): (1378, 1217),
-    (7, 400, 128, 0): (1385, 1603), (7, 513, 128, 0): (2026, 1948), (7, 600, 128, 0): (2055, 2007),
-    (7, 768, 128, 0): (2107, 2342), (7, 1003, 128, 0): (2668, 3036),
+    (5, 2300, 128, 0): (5923, 6507), (6, 1, 128, 0): (725, 719), (6, 8, 128, 0): (773, 742),
+    (6, 64, 128, 0): (785, 801), (6, 128, 128, 0): (797, 861), (6, 192, 128, 0): (792, 1148),
+    (6, 256, 128, 0): (812, 825), (6, 257, 128, 0): (1378, 1187), (6, 300, 128, 0): (1444, 1173),
+    (6, 400, 128, 0): (1447, 1515), (6, 513, 128, 0): (2064, 1887), (6, 600, 128, 0): (2119, 1889),
+    (6, 768, 128, 0): (2097, 2299), (6, 1003, 128, 0): (2734, 3001),
+    (6, 1200, 128, 0): (3365, 3694), (6, 1500, 128, 0): (4053, 4449),
+    (6, 2300, 128, 0): (6180, 6767), (7, 1, 128, 0): (741, 732), (7, 8, 128, 0): (783, 744),
+    (7, 64, 128, 0): (812, 792), (7, 128, 128, 0): (811, 838), (7, 192, 128, 0): (817, 1162),
+    (7, 256, 128, 0): (807, 838), (7, 257, 128, 0): (1386, 1197), (7, 300, 128, 0): (1495, 1180),
+    (7, 400, 128, 0): (1494, 1547), (7, 513, 128, 0): (2103, 1886), (7, 600, 128, 0): (2138, 1915),
+    (7, 768, 128, 0): (2107, 2342), (7, 1003, 128, 0): (2732, 3014),
     (7, 1200, 128, 0): (3435, 3728), (7, 1500, 128, 0): (4113, 4491),
-    (7, 2300, 128, 0): (6281, 6775), (4, 600, 128, 16): (1455, 1438),
-    (5, 600, 128, 16): (1491, 1550), (7, 600, 128, 16): (1610, 1655),
+    (7, 2300, 128, 0): (6281, 6775),
 }
 
 
@@ -140,9 +157,11 @@ def test_fused_choice_against_measured_times(route):
 
 
 def test_fused_only_where_rounds_count(route):
-    """Not up to one sequence per CU, nor from 16; any CU count is taken."""
+    """Up to one sequence per CU at a third of them and below, not from 16;
+    any CU count is taken."""
     for K in MAX_T:
         for ncu in (1, 3, NCU):
-            ns = [1, ncu, 16 * ncu, 40 * ncu]
+            ns = [ncu // 3 + 1, ncu, 16 * ncu, 40 * ncu]
             assert route([("f", K, MAX_T[K], n, ncu, 128, 256, ROW_BYTES[K]) for n in ns]) == [0] * 4
+        assert route([("f", K, MAX_T[K], n, NCU, 128, 256, ROW_BYTES[K]) for n in (1, 85)]) == [1] * 2
     assert route([("f", 4, 4, 5, 0, 128, 256, 2048)]) in ([0], [1])
