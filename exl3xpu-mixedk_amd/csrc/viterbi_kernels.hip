@@ -36,6 +36,8 @@
 // kernel only; every other kernel measured slower under it).
 #include "viterbi_kernels.h"
 
+#include <type_traits>
+
 #pragma clang fp contract(off)
 
 
@@ -320,6 +322,15 @@ struct FwdSmem {
     double red[kFwdThreads / 64];
 };
 
+// How fwd_run takes its count of sequences.  At T = 1 every caller passes 1: by
+// value the compiler puts that constant into fwd_run before inlining it, and
+// orders the column chain's steps less well for it (2560x4096 at K = 2 / 6:
+// 114.0 / 106.9 -> 114.5 / 107.4 ms, the other K within 0.2 %); by reference it
+// becomes a constant in each caller.  K = 3, whose plain forward has a unit of its
+// own, stays by value, as its column chain was measured.
+template <int K, int T>
+using CountArg = std::conditional_t<T == 1 && K != 3, const int&, int>;
+
 // Forward DP of sequences q0 .. q0+ntile-1 (ntile <= T) in lockstep by one
 // 1024-thread workgroup (the codebook registers are shared by the T
 // sequences; one barrier per step).  The caller fills sm.ovs[0..T) before
@@ -329,8 +340,8 @@ struct FwdSmem {
 // task loop and kept live across it).
 template <int K, int T>
 __device__ __forceinline__ void fwd_run(
-    FwdSmem<K, T>& sm, const float* __restrict__ X, int xstride, int xlen, int q0, int ntile,
-    const float* __restrict__ lut, int roll, int nsteps, int store_lo, bool pinned,
+    FwdSmem<K, T>& sm, const float* __restrict__ X, int xstride, int xlen, int q0,
+    CountArg<K, T> ntile, const float* __restrict__ lut, int roll, int nsteps, int store_lo, bool pinned,
     uint8_t* __restrict__ bp, int32_t* send, uint32_t* __restrict__ err, int tid) {
     using G = Geom<K>;
     auto& bbuf = sm.bbuf;
