@@ -162,8 +162,9 @@ __global__ __launch_bounds__(256, 2) void had_right_kernel(const float* __restri
 // read and one write 0.13 ms), to which the divisions, the LDS round trip and
 // the four barriers of a block add.  to_inner + from_inner, against the two
 // passes with the scales folded in that this replaces / against separate passes
-// for the scales too: 17408x5120 975 / 2965 -> 876 us, 4096x4096 211 / 460 ->
-// 178, 1024x1024 76 / 104 -> 52 (host side of two calls).
+// for the scales too: 17408x5120 975 / 2965 -> 876 us (876 to 1012 by the
+// device's clock), 4096x4096 211 / 460 -> 178, 1024x1024 76 / 104 -> 52 (host
+// side of two calls).
 template <bool DIV, bool MUL>
 __global__ __launch_bounds__(512, 2) void had_both_kernel(
     const float* __restrict__ hm, const float* __restrict__ in, float* __restrict__ out,
